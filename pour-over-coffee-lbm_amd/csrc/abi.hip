@@ -857,7 +857,7 @@ int pol_field_stats(pol_ctx* c, const pol_stats_opts* o, double* out, double* z_
   if (e == hipSuccess) e = launch_field_stats(d.storage == POL_F64, s, c->stat_dev, c->stat_dev + POL_NSTAT, st);
   if (e == hipSuccess && o->with_populations) {
     const StepArgs a = make_args(c, c->b.f[c->cur], nullptr, 0u);
-    e = launch_pop_nonfinite(d.storage, a, c->partial, c->stat_dev, c->wgrid, st);
+    e = launch_pop_nonfinite(d.storage, a, c->stat_dev, c->wgrid, st);
   }
   // one transfer of statistics and profile into pinned memory, then host copies
   const size_t nstat = (size_t)POL_NSTAT + (z_profile ? d.nz : 0);
