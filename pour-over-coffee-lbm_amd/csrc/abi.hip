@@ -25,6 +25,7 @@ struct pol_ctx {
   uint32_t part_cap = 0;  // blocks the partial buffers hold (any work grid fits)
   double* partial = nullptr;  // [nblk][POL_NRED]
   double* red_dev = nullptr;  // [POL_NRED]
+  double* host = nullptr;     // pinned [POL_NSTAT + nz]: results on their way to the caller
   // particles
   bool particles = false;
   bool pcoupled = false;  // the implicit drag field holds the footprint of a coupling
@@ -40,7 +41,6 @@ struct pol_ctx {
   double* stat_partial = nullptr;   // [nz * stat_tiles][POL_NSTAT]
   double* stat_zpart = nullptr;     // [nz * stat_tiles]
   double* stat_dev = nullptr;       // [POL_NSTAT + nz]
-  double* stat_host = nullptr;      // pinned copy of stat_dev (one transfer per call)
   // multiphase phase field
   bool mp = false;
   pol_multiphase_desc md{};
@@ -149,9 +149,9 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
   if (e == hipSuccess) e = hipMalloc((void**)&c->stat_partial, sblk * POL_NSTAT * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&c->stat_zpart, sblk * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&c->stat_dev, ((size_t)POL_NSTAT + d.nz) * sizeof(double));
-  if (e == hipSuccess) e = hipHostMalloc((void**)&c->stat_host, ((size_t)POL_NSTAT + d.nz) * sizeof(double));
+  if (e == hipSuccess) e = hipHostMalloc((void**)&c->host, ((size_t)POL_NSTAT + d.nz) * sizeof(double));
   if (e != hipSuccess) {
-    (void)hipHostFree(c->stat_host);
+    (void)hipHostFree(c->host);
     (void)hipFree(c->partial);
     (void)hipFree(c->red_dev);
     (void)hipFree(c->adj_partial);
@@ -176,7 +176,7 @@ int pol_destroy(pol_ctx* c) {
   (void)hipFree(c->stat_partial);
   (void)hipFree(c->stat_zpart);
   (void)hipFree(c->stat_dev);
-  (void)hipHostFree(c->stat_host);
+  (void)hipHostFree(c->host);
   delete c;
   return POL_OK;
 }
@@ -351,10 +351,13 @@ static int check_what(pol_ctx* c, uint32_t what, double* red_out, const char* fn
 }
 
 static int finish_reduce(pol_ctx* c, double* red_out, hipStream_t s, const char* fn) {
-  hipError_t e = launch_reduce_final(c->partial, c->wgrid.nblk, c->red_dev, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(red_out, c->red_dev, POL_NRED * sizeof(double), hipMemcpyDeviceToHost, s);
+  // the fold writes its 12 values straight into pinned host memory: a copy
+  // behind it would cost another 4 us of device time and its launch
+  hipError_t e = launch_reduce_final(c->partial, c->wgrid.nblk, c->host, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  return e == hipSuccess ? POL_OK : hip_fail(c, e, fn);
+  if (e != hipSuccess) return hip_fail(c, e, fn);
+  std::memcpy(red_out, c->host, POL_NRED * sizeof(double));
+  return POL_OK;
 }
 
 // The reference's finite-difference eddy viscosity from the velocity u
@@ -861,11 +864,11 @@ int pol_field_stats(pol_ctx* c, const pol_stats_opts* o, double* out, double* z_
   }
   // one transfer of statistics and profile into pinned memory, then host copies
   const size_t nstat = (size_t)POL_NSTAT + (z_profile ? d.nz : 0);
-  if (e == hipSuccess) e = hipMemcpyAsync(c->stat_host, c->stat_dev, nstat * sizeof(double), hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(c->host, c->stat_dev, nstat * sizeof(double), hipMemcpyDeviceToHost, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) return hip_fail(c, e, "pol_field_stats");
-  std::memcpy(out, c->stat_host, POL_NSTAT * sizeof(double));
-  if (z_profile) std::memcpy(z_profile, c->stat_host + POL_NSTAT, (size_t)d.nz * sizeof(double));
+  std::memcpy(out, c->host, POL_NSTAT * sizeof(double));
+  if (z_profile) std::memcpy(z_profile, c->host + POL_NSTAT, (size_t)d.nz * sizeof(double));
   return POL_OK;
 }
 

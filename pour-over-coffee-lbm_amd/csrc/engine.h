@@ -68,8 +68,9 @@ hipError_t launch_stream_collide(int storage, const StepArgs& a, bool store_f, c
 // Collisionless streaming pass a.fin -> a.fout (the step's gather, bounce-back
 // links, open faces and stores, no collision, no moments).
 hipError_t launch_stream_only(int storage, const StepArgs& a, const Grid& g, hipStream_t s);
-// Fold per-block partials into out[POL_NRED] (device), deterministic order.
-hipError_t launch_reduce_final(const double* partial, uint32_t nblk, double* out, hipStream_t s);
+// Fold per-block partials into out[POL_NRED] (device), deterministic order;
+// the partials are overwritten.
+hipError_t launch_reduce_final(double* partial, uint32_t nblk, double* out, hipStream_t s);
 // f = feq(rho, u) (rho/u real-typed, may be null); a.records selects the
 // compact layout (a.fout = f, a.N, a.P, a.n_items, a.cshift, a.dnx, a.nx used)
 hipError_t launch_init_equilibrium(int storage, const StepArgs& a, const void* rho, const void* u, const Grid& g,

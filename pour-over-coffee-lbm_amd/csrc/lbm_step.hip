@@ -20,31 +20,34 @@
 
 namespace pol {
 
-__global__ void __launch_bounds__(256) k_reduce_final(const double* __restrict__ partial, uint32_t nblk,
-                                                      double* __restrict__ out) {
-  __shared__ double sh[4][POL_NRED];
-  double v[POL_NRED];
-#pragma unroll
-  for (int s = 0; s < POL_NRED; ++s) v[s] = red_identity(s);
-  for (uint32_t b = threadIdx.x; b < nblk; b += 256) {
-#pragma unroll
-    for (int s = 0; s < POL_NRED; ++s) {
-      const double p = partial[(size_t)b * POL_NRED + s];
-      v[s] = red_is_max(s) ? fmax(v[s], p) : (red_is_min(s) ? fmin(v[s], p) : v[s] + p);
-    }
+// Fold of the per-block partials [rows][POL_NRED] (rows `stride` apart), in a
+// fixed order: block b folds rows [b per, (b + 1) per).  12 lanes read one
+// row, so a block's loads are whole lines; sub-row j takes rows j, j + 21, ...
+// and the 21 sub-rows meet in order.  One block over every row is bound by
+// the load rate of one CU (14 784 rows of the 224^3 cup: 28 us), so
+// launch_reduce_final folds more than FOLD_ROWS rows in two launches: up to
+// FOLD_ROWS blocks leave each its own first row (read by no other block) as
+// the sum of its rows, then one block folds those.
+constexpr uint32_t FOLD_SUB = 21;  // 21 x 12 = 252 lanes
+constexpr uint32_t FOLD_ROWS = 256;
+__global__ void __launch_bounds__(256) k_reduce_fold(double* partial, uint32_t rows, uint32_t stride, uint32_t per,
+                                                     double* out) {
+  __shared__ double sh[FOLD_SUB][POL_NRED];
+  const uint32_t s = threadIdx.x % POL_NRED, j = threadIdx.x / POL_NRED;
+  const bool is_max = red_is_max((int)s), is_min = red_is_min((int)s);
+  const uint32_t first = blockIdx.x * per, last = min(first + per, rows);
+  double v = red_identity((int)s);
+  auto add = [&](double r, double p) { return is_max ? fmax(r, p) : (is_min ? fmin(r, p) : r + p); };
+  if (j < FOLD_SUB) {
+#pragma unroll 4
+    for (uint32_t b = first + j; b < last; b += FOLD_SUB) v = add(v, partial[(size_t)b * stride * POL_NRED + s]);
+    sh[j][s] = v;
   }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int s = 0; s < POL_NRED; ++s) {
-    const double r = red_is_max(s) ? wave_max(v[s]) : (red_is_min(s) ? wave_min(v[s]) : wave_sum(v[s]));
-    if (lane == 0) sh[wid][s] = r;
-  }
-  __syncthreads();
+  __syncthreads();  // also: every row of this block has been read
   if (threadIdx.x < POL_NRED) {
-    const int s = threadIdx.x;
     double r = sh[0][s];
-    for (int w = 1; w < 4; ++w) r = red_is_max(s) ? fmax(r, sh[w][s]) : (red_is_min(s) ? fmin(r, sh[w][s]) : r + sh[w][s]);
-    out[s] = r;
+    for (uint32_t k = 1; k < FOLD_SUB; ++k) r = add(r, sh[k][s]);
+    (out ? out : partial + (size_t)first * stride * POL_NRED)[s] = r;
   }
 }
 
@@ -192,8 +195,18 @@ hipError_t launch_stream_only(int storage, const StepArgs& a, const Grid& g, hip
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_reduce_final(const double* partial, uint32_t nblk, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, s, partial, nblk, out);
+hipError_t launch_reduce_final(double* partial, uint32_t nblk, double* out, hipStream_t s) {
+  uint32_t rows = nblk, stride = 1;
+  // two launches pay from about 2 FOLD_ROWS rows on (one block: 512 rows take
+  // 5 us, the second launch about 4)
+  if (rows > 2 * FOLD_ROWS) {
+    stride = (nblk + FOLD_ROWS - 1) / FOLD_ROWS;
+    rows = (nblk + stride - 1) / stride;
+    hipLaunchKernelGGL(k_reduce_fold, dim3(rows), dim3(256), 0, s, partial, nblk, 1u, stride, nullptr);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k_reduce_fold, dim3(1), dim3(256), 0, s, partial, rows, stride, rows, out);
   return hipGetLastError();
 }
 
