@@ -13,9 +13,9 @@
 // to itself when x - e_q lies outside the box -- the reference's boundary
 // rule, every destination written exactly once.  A second kernel forms the
 // new temperature (the reference's compute_temperature) with the stability
-// test fused in; in a run of pure-diffusion steps each later collide pass
-// stores the temperature of its input state instead, and the second kernel
-// runs once, after the last step.  Temperature buffers ping-pong, so
+// test fused in; in a run of pure-diffusion steps the second kernel runs
+// once, after the last step, and the last collide pass stores the
+// temperature of its input state.  Temperature buffers ping-pong, so
 // temperature_old needs no copy.  The arithmetic follows the reference's FP32 expressions operation by
 // operation with contraction off:
 //   T = ((((((0 + g0) + g1) + g2) + g3) + g4) + g5) + g6
@@ -54,7 +54,8 @@ __device__ inline void decompose(const ThermalArgs& a, uint32_t i, uint32_t& x, 
 
 // WT: also store T = sum_q g_q of the input state into its temperature slot
 // (a.T) -- the value the previous step's temperature pass would have
-// written, so a run of pure-diffusion steps needs that pass only once.
+// written.  In a run of pure-diffusion steps only the last step does so (its
+// input state's temperature is the one a caller can still read afterwards).
 template <typename R, bool CONV, bool WT = false>
 __global__ void __launch_bounds__(256) k_thermal_collide(const ThermalArgs a) {
 #pragma clang fp contract(off)
@@ -275,11 +276,13 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
                                 int nsteps, hipStream_t s) {
   // With convection a step's source needs the whole temperature field of its
   // input state before it starts, so every step runs the temperature pass.
-  // Pure diffusion reads only the cell's own populations: the collide pass of
-  // step n + 1 stores T of its input state (state n + 1) itself, and the
-  // temperature pass (with the stability test that is reported) runs after
-  // the last step only.  The first step leaves the input state's temperature
-  // as the caller set it (it may be a boundary value rather than sum g).
+  // Pure diffusion reads only the cell's own populations: the temperature
+  // pass (with the stability test that is reported) runs after the last step
+  // only, and the last step's collide pass stores T of its input state
+  // itself.  The steps between store none (two temperature buffers: each
+  // would be overwritten unread, 4 of 64 B per cell).  A run's first step
+  // leaves the input state's temperature as the caller set it (it may be a
+  // boundary value rather than sum g).
   const dim3 grid((base.N + 255) / 256);
   for (int n = 0; n < nsteps; ++n) {
     ThermalArgs a = base;
@@ -290,7 +293,7 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
     const bool last = n + 1 == nsteps;
     if (a.conv)
       hipLaunchKernelGGL((k_thermal_collide<R, true>), grid, dim3(256), 0, s, a);
-    else if (n == 0)
+    else if (n == 0 || !last)
       hipLaunchKernelGGL((k_thermal_collide<R, false>), grid, dim3(256), 0, s, a);
     else
       hipLaunchKernelGGL((k_thermal_collide<R, false, true>), grid, dim3(256), 0, s, a);
