@@ -551,6 +551,11 @@ int pol_thermal_step(pol_ctx *ctx, int nsteps, int32_t *unstable_out, void *stre
 int pol_thermal_heat_flux(pol_ctx *ctx, void *flux, void *stream);
 /* {min, max, sum} of the current temperature (FP64, host); synchronous. */
 int pol_thermal_stats(pol_ctx *ctx, double *out3, void *stream);
+/* The figures of the coupled loop's stability check in one pass
+ * (thermal_fluid_coupled.py:237-262): {min, max, sum} of the current
+ * temperature and the number of cells whose bound velocity has |u| > 1 (FP64,
+ * host); synchronous. */
+int pol_thermal_coupling_stats(pol_ctx *ctx, double *out4, void *stream);
 /* Boundary forms of thermal_lbm.py:288-346 on the cells where mask (uint8
  * [cells]) is non-zero: kind 1 Dirichlet (T = a, g = w a), kind 2 Neumann
  * (S = a), kind 3 convective (S = -a (T - b)). */

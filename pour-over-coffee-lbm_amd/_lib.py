@@ -228,6 +228,7 @@ SIGNATURES = {
     "pol_thermal_step": (C.c_int, [_P, C.c_int, _P, _P]),
     "pol_thermal_heat_flux": (C.c_int, [_P, _P, _P]),
     "pol_thermal_stats": (C.c_int, [_P, _P, _P]),
+    "pol_thermal_coupling_stats": (C.c_int, [_P, _P, _P]),
     "pol_thermal_boundary": (C.c_int, [_P, C.c_int, _P, C.c_double, C.c_double, _P]),
     "pol_multiphase_bind": (C.c_int, [_P, C.POINTER(PolMultiphaseDesc), C.POINTER(PolMultiphaseBuffers)]),
     "pol_multiphase_chemical_potential": (C.c_int, [_P, _P, _P]),

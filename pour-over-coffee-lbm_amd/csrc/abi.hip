@@ -24,7 +24,7 @@ struct pol_ctx {
   uint32_t P = 0;         // population plane stride (N, or the compact layout's stored cells)
   uint32_t part_cap = 0;  // blocks the partial buffers hold (any work grid fits)
   double* partial = nullptr;  // [nblk][POL_NRED]
-  double* red_dev = nullptr;  // [POL_NRED]
+  uint32_t* bad_dev = nullptr;  // [1] cells failing the thermal stability test
   double* host = nullptr;     // pinned [POL_NSTAT + nz]: results on their way to the caller
   // particles
   bool particles = false;
@@ -134,7 +134,7 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
   c->part_cap = make_grid((uint64_t)d.ny * d.nz * ((uint64_t)d.nx + 63)).nblk;
   hipError_t e = hipSetDevice(d.device);
   if (e == hipSuccess) e = hipMalloc((void**)&c->partial, (size_t)c->part_cap * POL_NRED * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void**)&c->red_dev, POL_NRED * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc((void**)&c->bad_dev, sizeof(uint32_t));
   if (e == hipSuccess) e = hipMalloc((void**)&c->adj_partial, (size_t)c->part_cap * 4 * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&c->adj_acc, 4 * sizeof(double));
   // statistics: up to 12 blocks per plane (2688 blocks at 224^3, each lane
@@ -153,7 +153,7 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
   if (e != hipSuccess) {
     (void)hipHostFree(c->host);
     (void)hipFree(c->partial);
-    (void)hipFree(c->red_dev);
+    (void)hipFree(c->bad_dev);
     (void)hipFree(c->adj_partial);
     (void)hipFree(c->adj_acc);
     (void)hipFree(c->stat_partial);
@@ -170,7 +170,7 @@ int pol_destroy(pol_ctx* c) {
   if (!c) return POL_OK;
   (void)hipSetDevice(c->d.device);
   (void)hipFree(c->partial);
-  (void)hipFree(c->red_dev);
+  (void)hipFree(c->bad_dev);
   (void)hipFree(c->adj_partial);
   (void)hipFree(c->adj_acc);
   (void)hipFree(c->stat_partial);
@@ -1167,7 +1167,7 @@ static ThermalArgs thermal_args(const pol_ctx* c) {
   a.omega_f = (float)c->td.omega;
   a.omega_d = c->td.omega;
   a.conv = (c->td.options & POL_THERMAL_CONVECTION) ? 1u : 0u;
-  a.partial = c->partial;
+  a.bad = c->bad_dev;
   return a;
 }
 
@@ -1231,11 +1231,10 @@ int pol_thermal_step(pol_ctx* c, int nsteps, int32_t* unstable_out, void* stream
     if (nsteps == 0) {
       *unstable_out = 0;
     } else {
-      e = launch_thermal_fold(c->partial, (c->N + 255) / 256, 1, c->red_dev, s);
-      double v = 0.0;
-      if (e == hipSuccess) e = hipMemcpyAsync(&v, c->red_dev, sizeof(double), hipMemcpyDeviceToHost, s);
+      uint32_t* v = (uint32_t*)c->host;
+      e = hipMemcpyAsync(v, c->bad_dev, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipStreamSynchronize(s);
-      *unstable_out = (int32_t)v;
+      if (e == hipSuccess) *unstable_out = (int32_t)*v;
     }
   }
   return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_thermal_step");
@@ -1249,17 +1248,28 @@ int pol_thermal_heat_flux(pol_ctx* c, void* flux, void* stream) {
   return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_thermal_heat_flux");
 }
 
-int pol_thermal_stats(pol_ctx* c, double* out3, void* stream) {
-  if (!c || !out3) return POL_ERR_INVALID;
-  if (!c->thermal) return fail(c, POL_ERR_STATE, "pol_thermal_stats: thermal buffers not bound");
+static int thermal_stats(pol_ctx* c, const void* u, double* out, int nval, void* stream, const char* where) {
+  if (!c->thermal) return fail(c, POL_ERR_STATE, std::string(where) + ": thermal buffers not bound");
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipSetDevice(c->d.device);
   if (e == hipSuccess)
-    e = launch_thermal_stats(c->d.storage == POL_F64, c->tb.temperature[c->tcur], c->N, c->partial, s);
-  if (e == hipSuccess) e = launch_thermal_fold(c->partial, (c->N + 255) / 256, 3, c->red_dev, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(out3, c->red_dev, 3 * sizeof(double), hipMemcpyDeviceToHost, s);
+    e = launch_thermal_stats(c->d.storage == POL_F64, c->tb.temperature[c->tcur], u, c->N, c->partial, c->host, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_thermal_stats");
+  if (e != hipSuccess) return hip_fail(c, e, where);
+  std::memcpy(out, c->host, nval * sizeof(double));
+  return POL_OK;
+}
+
+int pol_thermal_stats(pol_ctx* c, double* out3, void* stream) {
+  if (!c || !out3) return POL_ERR_INVALID;
+  return thermal_stats(c, nullptr, out3, 3, stream, "pol_thermal_stats");
+}
+
+int pol_thermal_coupling_stats(pol_ctx* c, double* out4, void* stream) {
+  if (!c || !out4) return POL_ERR_INVALID;
+  if (c->thermal && !c->tb.velocity)
+    return fail(c, POL_ERR_INVALID, "pol_thermal_coupling_stats: needs the velocity buffer");
+  return thermal_stats(c, c->tb.velocity, out4, 4, stream, "pol_thermal_coupling_stats");
 }
 
 int pol_thermal_boundary(pol_ctx* c, int kind, const uint8_t* mask, double a, double b, void* stream) {

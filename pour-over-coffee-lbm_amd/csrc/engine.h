@@ -179,14 +179,16 @@ struct ThermalArgs {
   float omega_f;
   double omega_d;
   uint32_t conv;
-  double* partial;   // per-block partials (stability counts, statistics)
+  uint32_t* bad;     // cells that fail the stability test of the last step
 };
 // nsteps steps ping-ponging g[gcur] / T[tcur]; base supplies the fields.
 hipError_t launch_thermal_steps(bool dbl, const ThermalArgs& base, void* const g[2], void* const T[2], int& gcur,
                                 int& tcur, int nsteps, hipStream_t s);
-// Fold per-block partials: nval 1 = sum into out[0]; 3 = {min, max, sum}.
-hipError_t launch_thermal_fold(const double* partial, uint32_t nblk, int nval, double* out, hipStream_t s);
-hipError_t launch_thermal_stats(bool dbl, const void* T, uint32_t N, double* partial, hipStream_t s);
+// {min, max, sum} of T and, where u (real [3][N]) is not null, the number of
+// cells with |u| > 1 (else 0) into out[4] (device or pinned host memory);
+// partial holds at least 4 x min(1024, ceil(N / 256)) doubles.
+hipError_t launch_thermal_stats(bool dbl, const void* T, const void* u, uint32_t N, double* partial, double* out,
+                                hipStream_t s);
 hipError_t launch_thermal_flux(bool dbl, const ThermalArgs& a, void* flux, hipStream_t s);
 hipError_t launch_thermal_init(bool dbl, const ThermalArgs& a, hipStream_t s);
 hipError_t launch_thermal_boundary(bool dbl, const ThermalArgs& a, int kind, const uint8_t* mask, double va,

@@ -26,6 +26,8 @@
 // (+ convection), and writes S to the heat source: the coupled loop's
 // reset_heat_source_to_base (thermal_fluid_coupled.py:193-194) at no extra
 // pass.
+#include <algorithm>
+
 #include "engine.h"
 
 namespace pol {
@@ -61,6 +63,7 @@ __global__ void __launch_bounds__(256) k_thermal_collide(const ThermalArgs a) {
 #pragma clang fp contract(off)
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i >= a.N) return;
+  if (i == 0) *a.bad = 0u;  // counted by the temperature pass that follows
   uint32_t x, y, z;
   decompose(a, i, x, y, z);
   const R* __restrict__ gin = (const R*)a.gin;
@@ -113,107 +116,122 @@ __global__ void __launch_bounds__(256) k_thermal_collide(const ThermalArgs a) {
   }
 }
 
-// T' = sum_q g'_q and the stability test, per-block counts of failing cells.
+// T' = sum_q g'_q and the stability test.  Bound by reading the populations
+// (224^3: 0.075 ms for 360 MB).  Failing cells are counted in *a.bad, which
+// the collide pass before has set to zero: a wave without one (every wave of
+// a stable state) neither reduces nor stores anything.  A count per block
+// would need a fold over 43 904 of them, 0.057 ms per step on one block.
 template <typename R>
 __global__ void __launch_bounds__(256) k_thermal_temperature(const ThermalArgs a) {
 #pragma clang fp contract(off)
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  double bad = 0.0;
-  if (i < a.N) {
-    const R* __restrict__ g = (const R*)a.gout;
-    const size_t N = a.N;
-    R T = R(0);
-    bool gbad = false;
+  if (i >= a.N) return;
+  const R* __restrict__ g = (const R*)a.gout;
+  const size_t N = a.N;
+  R T = R(0);
+  bool bad = false;
 #pragma unroll
-    for (int q = 0; q < TQ; ++q) {
-      const R v = g[q * N + i];
-      T = T + v;
-      gbad = gbad || !(v == v) || fabs(v) > R(1000);
-    }
-    ((R*)a.Tout)[i] = T;
-    if (T < R(-50) || T > R(150) || !(T == T) || gbad) bad = 1.0;
+  for (int q = 0; q < TQ; ++q) {
+    const R v = g[q * N + i];
+    T = T + v;
+    bad = bad || !(v == v) || fabs(v) > R(1000);
   }
-  bad = wave_sum(bad);
-  __shared__ double sh[4];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) sh[wid] = bad;
-  __syncthreads();
-  if (threadIdx.x == 0) a.partial[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  ((R*)a.Tout)[i] = T;
+  bad = bad || T < R(-50) || T > R(150) || !(T == T);
+  const uint64_t cells = __ballot(bad);
+  // the lowest failing lane adds the wave's count
+  if (bad && (cells & ((1ull << (threadIdx.x & 63)) - 1ull)) == 0ull) atomicAdd(a.bad, (uint32_t)__popcll(cells));
 }
 
-__global__ void __launch_bounds__(256) k_thermal_fold(const double* __restrict__ partial, uint32_t nblk, int nval,
-                                                      double* __restrict__ out) {
-  // nval = 1: sum; nval = 3: {min, max, sum} triples
-  __shared__ double sh[4][3];
-  double v[3] = {1.0e300, -1.0e300, 0.0};
-  if (nval == 1) v[2] = 0.0;
-  for (uint32_t b = threadIdx.x; b < nblk; b += 256) {
-    if (nval == 1) {
-      v[2] += partial[b];
-    } else {
-      v[0] = fmin(v[0], partial[(size_t)b * 3]);
-      v[1] = fmax(v[1], partial[(size_t)b * 3 + 1]);
-      v[2] += partial[(size_t)b * 3 + 2];
-    }
-  }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  v[0] = wave_min(v[0]);
-  v[1] = wave_max(v[1]);
-  v[2] = wave_sum(v[2]);
-  if (lane == 0) {
-    sh[wid][0] = v[0];
-    sh[wid][1] = v[1];
-    sh[wid][2] = v[2];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double r0 = sh[0][0], r1 = sh[0][1], r2 = sh[0][2];
-    for (int w = 1; w < 4; ++w) {
-      r0 = fmin(r0, sh[w][0]);
-      r1 = fmax(r1, sh[w][1]);
-      r2 += sh[w][2];
-    }
-    if (nval == 1) {
-      out[0] = r2;
-    } else {
-      out[0] = r0;
-      out[1] = r1;
-      out[2] = r2;
-    }
-  }
-}
+// {min, max, sum} of T and, with a velocity, the number of cells with |u| > 1:
+// up to STAT_BLOCKS blocks stride over the field, four values a lane and load
+// where the field's size allows it, and keep their lanes' results in
+// registers, so the field is read at memory speed and 1024 rows are left to
+// fold.  (One value a lane with a row per 256 cells was bound by its FP64
+// shuffles: 0.074 ms for 45 MB, and 0.057 ms to fold 43 904 rows.)
+constexpr uint32_t STAT_BLOCKS = 1024;
+constexpr int STAT_ROW = 4;
 
 template <typename R>
-__global__ void __launch_bounds__(256) k_thermal_stats(const R* __restrict__ T, uint32_t N, double* __restrict__ partial) {
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  double mn = 1.0e300, mx = -1.0e300, sm = 0.0;
-  if (i < N) {
-    const double t = (double)T[i];
-    mn = t;
-    mx = t;
-    sm = t;
+__device__ inline void load_quad(const R* __restrict__ p, uint32_t j, R (&v)[4]) {
+  if constexpr (sizeof(R) == 4) {
+    const float4 t = ((const float4*)p)[j];
+    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+  } else {
+    const double2 t0 = ((const double2*)p)[2 * (size_t)j], t1 = ((const double2*)p)[2 * (size_t)j + 1];
+    v[0] = t0.x; v[1] = t0.y; v[2] = t1.x; v[3] = t1.y;
   }
+}
+
+template <typename R, int W>
+__global__ void __launch_bounds__(256) k_thermal_stats(const R* __restrict__ T, const R* __restrict__ u, uint32_t N,
+                                                       double* __restrict__ partial) {
+#pragma clang fp contract(off)
+  double mn = 1.0e300, mx = -1.0e300, sm = 0.0;
+  uint32_t fast = 0;
+  const uint32_t items = N / W;
+  auto one = [&](R t) {
+    const double d = (double)t;
+    mn = fmin(mn, d);
+    mx = fmax(mx, d);
+    sm += d;
+  };
+  auto speed = [&](R x, R y, R z) { fast += sqrt((x * x + y * y) + z * z) > R(1) ? 1u : 0u; };
+  for (uint32_t j = blockIdx.x * 256u + threadIdx.x; j < items; j += gridDim.x * 256u) {
+    if constexpr (W == 4) {
+      R t[4];
+      load_quad<R>(T, j, t);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) one(t[k]);
+      if (u) {
+        R x[4], y[4], z[4];
+        load_quad<R>(u, j, x);
+        load_quad<R>(u + N, j, y);
+        load_quad<R>(u + 2 * (size_t)N, j, z);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) speed(x[k], y[k], z[k]);
+      }
+    } else {
+      one(T[j]);
+      if (u) speed(u[j], u[(size_t)N + j], u[2 * (size_t)N + j]);
+    }
+  }
+  double c = (double)fast;
   mn = wave_min(mn);
   mx = wave_max(mx);
   sm = wave_sum(sm);
-  __shared__ double sh[4][3];
+  c = wave_sum(c);
+  __shared__ double sh[4][STAT_ROW];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if (lane == 0) {
     sh[wid][0] = mn;
     sh[wid][1] = mx;
     sh[wid][2] = sm;
+    sh[wid][3] = c;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double r0 = sh[0][0], r1 = sh[0][1], r2 = sh[0][2];
-    for (int w = 1; w < 4; ++w) {
-      r0 = fmin(r0, sh[w][0]);
-      r1 = fmax(r1, sh[w][1]);
-      r2 += sh[w][2];
-    }
-    partial[(size_t)blockIdx.x * 3] = r0;
-    partial[(size_t)blockIdx.x * 3 + 1] = r1;
-    partial[(size_t)blockIdx.x * 3 + 2] = r2;
+  if (threadIdx.x < STAT_ROW) {
+    const int s = threadIdx.x;
+    double r = sh[0][s];
+    for (int w = 1; w < 4; ++w) r = s == 0 ? fmin(r, sh[w][s]) : (s == 1 ? fmax(r, sh[w][s]) : r + sh[w][s]);
+    partial[(size_t)blockIdx.x * STAT_ROW + s] = r;
+  }
+}
+
+// Fold of at most STAT_BLOCKS rows {min, max, sum, count} into out (pinned host memory)
+__global__ void __launch_bounds__(256) k_thermal_fold(const double* __restrict__ partial, uint32_t rows,
+                                                      double* __restrict__ out) {
+  __shared__ double sh[64][STAT_ROW];
+  const int s = threadIdx.x & 3, j = threadIdx.x >> 2;
+  auto add = [&](double r, double p) { return s == 0 ? fmin(r, p) : (s == 1 ? fmax(r, p) : r + p); };
+  double v = s == 0 ? 1.0e300 : (s == 1 ? -1.0e300 : 0.0);
+  for (uint32_t b = j; b < rows; b += 64) v = add(v, partial[(size_t)b * STAT_ROW + s]);
+  sh[j][s] = v;
+  __syncthreads();
+  if (threadIdx.x < STAT_ROW) {
+    double r = sh[0][threadIdx.x];
+    for (int k = 1; k < 64; ++k) r = add(r, sh[k][threadIdx.x]);
+    out[threadIdx.x] = r;
   }
 }
 
@@ -312,18 +330,26 @@ hipError_t launch_thermal_steps(bool dbl, const ThermalArgs& base, void* const g
              : thermal_steps<float>(base, g, T, gcur, tcur, nsteps, s);
 }
 
-hipError_t launch_thermal_fold(const double* partial, uint32_t nblk, int nval, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_thermal_fold, dim3(1), dim3(256), 0, s, partial, nblk, nval, out);
+template <typename R>
+static hipError_t thermal_stats(const void* T, const void* u, uint32_t N, double* partial, double* out, hipStream_t s) {
+  // four values a load when every component of u starts on a 16-byte
+  // boundary (N % 4; the bases are allocations or whole multiples of it)
+  const bool quad = N % 4 == 0 && ((uintptr_t)T & 15) == 0 && ((uintptr_t)u & 15) == 0;
+  const uint32_t items = quad ? N / 4 : N;
+  const uint32_t blocks = std::min((items + 255u) / 256u, STAT_BLOCKS);
+  if (quad)
+    hipLaunchKernelGGL((k_thermal_stats<R, 4>), dim3(blocks), dim3(256), 0, s, (const R*)T, (const R*)u, N, partial);
+  else
+    hipLaunchKernelGGL((k_thermal_stats<R, 1>), dim3(blocks), dim3(256), 0, s, (const R*)T, (const R*)u, N, partial);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_thermal_fold, dim3(1), dim3(256), 0, s, partial, blocks, out);
   return hipGetLastError();
 }
 
-hipError_t launch_thermal_stats(bool dbl, const void* T, uint32_t N, double* partial, hipStream_t s) {
-  const dim3 grid((N + 255) / 256);
-  if (dbl)
-    hipLaunchKernelGGL(k_thermal_stats<double>, grid, dim3(256), 0, s, (const double*)T, N, partial);
-  else
-    hipLaunchKernelGGL(k_thermal_stats<float>, grid, dim3(256), 0, s, (const float*)T, N, partial);
-  return hipGetLastError();
+hipError_t launch_thermal_stats(bool dbl, const void* T, const void* u, uint32_t N, double* partial, double* out,
+                                hipStream_t s) {
+  return dbl ? thermal_stats<double>(T, u, N, partial, out, s) : thermal_stats<float>(T, u, N, partial, out, s);
 }
 
 hipError_t launch_thermal_flux(bool dbl, const ThermalArgs& a, void* flux, hipStream_t s) {

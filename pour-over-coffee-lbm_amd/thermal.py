@@ -427,14 +427,17 @@ class ThermalFluidCoupledSolver:
         return True
 
     def _check_coupling_stability(self) -> bool:
-        """thermal_fluid_coupled.py:237-262 (the velocity bound on the device)."""
-        tmin, tmax, _ = self.thermal_solver.get_temperature_stats()
+        """thermal_fluid_coupled.py:237-262, its figures from one device pass."""
+        th = self.thermal_solver
+        out = np.zeros(4, dtype=np.float64)
+        L.check(th.lib.pol_thermal_coupling_stats(th.ctx.handle, out.ctypes.data, L.stream_handle()), th.ctx.handle,
+                "pol_thermal_coupling_stats")
+        tmin, tmax, _, fast_cells = (float(v) for v in out)
         if tmax > 150.0 or tmin < -10.0:
             return False
         if abs(tmax - tmin) > self.coupling_config.max_coupling_error:
             return False
-        u = self.thermal_solver._vel
-        return not bool((torch.linalg.vector_norm(u, dim=0) > 1.0).any())
+        return fast_cells == 0
 
     def get_coupling_diagnostics(self) -> dict:
         """thermal_fluid_coupled.py:264-304."""

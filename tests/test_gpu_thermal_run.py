@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from pourover_amd.thermal import ThermalLBM
+from pourover_amd.thermal import ThermalFluidCoupledSolver, ThermalLBM
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +44,50 @@ def test_run_equals_single_steps(shape, precision, convection):
         for name in ("temperature", "temperature_old", "heat_source"):
             assert torch.equal(getattr(a, name).to_torch(), getattr(b, name).to_torch()), name
         assert torch.equal(a.g_device, b.g_device)
+
+
+@pytest.mark.parametrize("precision", ["f32", "f64"])
+@pytest.mark.parametrize("shape", SHAPES + [(128, 64, 33), (101, 103, 107)])
+def test_statistics(shape, precision):
+    print("case: thermal statistics %s %s" % (shape, precision), flush=True)
+    th = _make(shape, precision, True)
+    T = th.temperature.to_torch().double().cpu().numpy()
+    n, eps = T.size, np.finfo(np.float64).eps
+    lo, hi, mean = th.get_temperature_stats()
+    assert lo == T.min() and hi == T.max()
+    assert abs(mean * n - T.sum()) <= n * eps * np.abs(T).sum() + 2 * eps * abs(mean * n)  # any order of the sum
+    coupled = ThermalFluidCoupledSolver(fluid_solver=_Fluid(), thermal_solver=th)
+    assert coupled._check_coupling_stability()
+    for at in (0, n // 2, n - 1):  # |u| > 1 in one cell, wherever it lies
+        th._vel.view(3, -1)[:, at] = torch.tensor([0.6, 0.6, -0.6])
+        assert not coupled._check_coupling_stability()
+        th._vel.view(3, -1)[:, at] = torch.tensor([float("nan"), 2.0, 0.0])  # as a norm of NaN: not above 1
+        assert coupled._check_coupling_stability()
+        th._vel.view(3, -1)[:, at] = torch.tensor([float("inf"), 0.0, 0.0])
+        assert not coupled._check_coupling_stability()
+        th._vel.view(3, -1)[:, at] = 0.0
+    th.temperature.to_torch().view(-1)[n - 1] = 151.0
+    assert not coupled._check_coupling_stability()
+    th.temperature.to_torch().view(-1)[n - 1] = -11.0
+    assert not coupled._check_coupling_stability()
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_count_of_unstable_cells(shape):
+    """0, 1, some and all cells outside the stability bounds, and afresh after each."""
+    n = shape[0] * shape[1] * shape[2]
+    for share in (0.0, 0.3, 1.0, 0.0):
+        th = _make(shape, "f32", False)
+        rng = np.random.default_rng(int(share * 10))
+        T = np.where(rng.random(shape) < share, np.float32(1e4), np.float32(50.0))
+        th.initialize_from(T)
+        ok = th.step()
+        g = th.g_device.cpu().numpy()
+        Tn = th.temperature.to_torch().cpu().numpy()
+        bad = (Tn < -50) | (Tn > 150) | (np.abs(g) > 1000).any(axis=0)
+        assert th._last_unstable == int(bad.sum()) and ok == (not bad.any())
+    assert n > 0
+
+
+class _Fluid:
+    """The coupled solver asks its fluid solver for nothing in these checks."""
