@@ -57,9 +57,7 @@ __device__ inline double combine_c(double a, double b) {
   else return a + b;
 }
 __device__ inline double wave_combine(int s, double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = stat_combine(s, v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_reduce(v, [s](double a, double b) { return stat_combine(s, a, b); });
 }
 
 // |u| in FP32 without contraction: ((ux*ux) + (uy*uy)) + (uz*uz), each
@@ -108,12 +106,10 @@ __host__ __device__ constexpr int stat_role(int s) {
 template <int S>
 __device__ inline void wave_stat(double v, uint32_t cnt, double (*sh)[POL_NSTAT + 1], int wid, int lane) {
   if constexpr (stat_is_count(S)) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
+    cnt = wave_reduce(cnt, [](uint32_t a, uint32_t b) { return a + b; });
     if (lane == 0) sh[wid][S] = (double)cnt;
   } else {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = combine_c<S>(v, __shfl_xor(v, o, 64));
+    v = wave_reduce(v, [](double a, double b) { return combine_c<S>(a, b); });
     if (lane == 0) sh[wid][S] = v;
   }
 }
@@ -169,11 +165,7 @@ __device__ inline double umag_of_key(uint32_t k) { return (double)__uint_as_floa
 // decoded: an empty key gives the statistic's identity, a NaN key NaN.
 template <int S, bool MIN>
 __device__ inline void wave_key(uint32_t k, double (*sh)[POL_NSTAT + 1], int wid, int lane) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint32_t t = __shfl_xor(k, o, 64);
-    k = MIN ? min(k, t) : max(k, t);
-  }
+  k = wave_reduce(k, [](uint32_t a, uint32_t b) { return MIN ? min(a, b) : max(a, b); });
   if (lane == 0) {
     const bool empty = MIN ? k == ~0u : k == 0u;
     sh[wid][S] = empty ? stat_identity(S) : (k > UKEY_INF ? (double)NAN : umag_of_key(k));
@@ -523,8 +515,7 @@ __global__ void __launch_bounds__(BLOCK) k_pop_nonfinite(const StepArgs a, doubl
     }
   }
   if (__ballot(bad != 0u) == 0ull) return;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) bad += __shfl_xor(bad, o, 64);
+  bad = wave_reduce(bad, [](uint32_t a, uint32_t b) { return a + b; });
   if ((threadIdx.x & 63) == 0) {
     if (bad & 0xffffu) unsafeAtomicAdd(out + POL_STAT_FLUID_POP_NAN, (double)(bad & 0xffffu));
     if (bad >> 16) unsafeAtomicAdd(out + POL_STAT_FLUID_POP_INF, (double)(bad >> 16));

@@ -317,22 +317,60 @@ constexpr uint32_t BOUNCE_BITS = 0x7fffeu;
 __device__ inline uint32_t slot_clamp(int s, uint32_t P) { return min((uint32_t)s, P - 1u); }
 
 // ---------------------------------------------------------------------------
-// wave64 reductions (DPP/permute via shfl_xor) in FP64
+// wave64 reductions without the LDS crossbar.  A __shfl_xor of a double is two
+// ds_bpermute_b32, the waves of a CU share one LDS pipe for them, and the
+// 12-slot reduction epilogue (144 of them) took a quarter of the moments pass.
+// lane_pair<O> gives a and b such that {a, b} = {v(lane), v(lane ^ O)}: within
+// a row of 16 lanes by DPP moves, across rows by gfx950's swaps (the swap of a
+// register with itself leaves the value of the lower half row / wave in one
+// result and that of the upper one in the other, in every lane).  O = 4
+// rotates a row by 4 instead of exchanging it: after the O = 8 step lanes i
+// and i ^ 8 hold the same value, so lane i - 4 holds what lane i ^ 4 does.
+// All 64 lanes must be active.
 // ---------------------------------------------------------------------------
+template <int O>
+__device__ inline void lane_pair(uint32_t v, uint32_t& a, uint32_t& b) {
+  if constexpr (O == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+  } else if constexpr (O == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+  } else {
+    constexpr int ctrl = O == 8 ? 0x128 /* row_ror:8 */ : O == 4 ? 0x124 /* row_ror:4 */
+                         : O == 2 ? 0x4e /* quad_perm:[2,3,0,1] */ : 0xb1 /* quad_perm:[1,0,3,2] */;
+    a = v;
+    b = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, ctrl, 0xf, 0xf, true);
+  }
+}
+template <int O>
+__device__ inline void lane_pair(double v, double& a, double& b) {
+  const uint64_t w = __builtin_bit_cast(uint64_t, v);
+  uint32_t alo, ahi, blo, bhi;
+  lane_pair<O>((uint32_t)w, alo, blo);
+  lane_pair<O>((uint32_t)(w >> 32), ahi, bhi);
+  a = __builtin_bit_cast(double, (uint64_t)alo | ((uint64_t)ahi << 32));
+  b = __builtin_bit_cast(double, (uint64_t)blo | ((uint64_t)bhi << 32));
+}
+// All 64 lanes' values combined by the commutative op, in every lane.
+template <int O = 32, typename T, typename Op>
+__device__ inline T wave_reduce(T v, Op&& op) {
+  T a, b;
+  lane_pair<O>(v, a, b);
+  v = op(a, b);
+  if constexpr (O > 1) return wave_reduce<O / 2>(v, op);
+  else return v;
+}
 __device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return wave_reduce(v, [](double a, double b) { return a + b; });
 }
 __device__ inline double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_reduce(v, [](double a, double b) { return fmax(a, b); });
 }
 __device__ inline double wave_min(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_reduce(v, [](double a, double b) { return fmin(a, b); });
 }
 
 // Per-block partials of the POL_NRED reduction slots.  Slots UMAX/RHOMAX
