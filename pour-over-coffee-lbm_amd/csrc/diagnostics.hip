@@ -252,10 +252,12 @@ struct StatsB {
   // Mach > 1e-10 | Mach > 0.1 << 16, |u| > 1e-10 | interior << 16,
   // NaN |u| | infinite |u| << 16 (non-solid cells)
   uint32_t c_mach = 0, c_um = 0, c_nonfinite = 0;
-  // i: the cell's index within plane z (base = z nxy); in_box: 1 <= x, y, z
-  // <= n - 2 (the interior test without the solid check)
+  // in_box: 1 <= x, y, z <= n - 2 (the interior test without the solid check)
+  // pr, px, py, pz, ph: the cell's previous density and velocity and its phase
+  // (EXTRA; read where the arguments have them)
   template <typename R>
-  __device__ void add(const StatsArgs& a, size_t base, uint32_t i, bool in_box, R r, R ux, R uy, R uz, uint32_t fl) {
+  __device__ void add(const StatsArgs& a, bool in_box, R r, R ux, R uy, R uz, uint32_t fl, R pr, R px, R py, R pz,
+                      R ph) {
     const double rd = (double)r;
     const float umf = umag_f32(ux, uy, uz);
     const double um = (double)umf;
@@ -273,16 +275,14 @@ struct StatsB {
     bool water = true;
     if constexpr (EXTRA) {
       if (a.prev_rho) {
-        const double e = rd - (double)((const R*)a.prev_rho)[base + i];
+        const double e = rd - (double)pr;
         p_r2 += e * e;
       }
       if (a.prev_u) {
-        const R* pu = (const R*)a.prev_u + base + i;
-        const double ex = (double)ux - (double)pu[0], ey = (double)uy - (double)pu[a.N],
-                     ez = (double)uz - (double)pu[2 * (size_t)a.N];
+        const double ex = (double)ux - (double)px, ey = (double)uy - (double)py, ez = (double)uz - (double)pz;
         p_u2 += ex * ex + ey * ey + ez * ez;
       }
-      if (a.phase) water = ((const R*)a.phase)[base + i] > R(0.1);
+      if (a.phase) water = ph > R(0.1);
     }
     const bool ns = ((fl >> POL_KIND_SHIFT) & POL_KIND_MASK) != POL_KIND_SOLID;
     c_nonfinite += (ns && key > UKEY_INF) ? 1u : 0u;
@@ -337,6 +337,26 @@ struct Group4 {
   }
 };
 
+// The previous density and velocity and the phase of four consecutive cells
+// (index i of the field; the launcher takes the 4-cell form only where each
+// of the given fields starts on a 16-byte boundary).  Loaded up front with
+// the cells' own values: read one by one behind the tests for each pointer
+// they took the pass from 0.063 to 0.143 ms (224^3, previous state given).
+template <typename R>
+struct Extra4 {
+  R pr[4], px[4], py[4], pz[4], ph[4];
+  __device__ void load(const StatsArgs& a, size_t i) {
+    if (a.prev_rho) load4((const R*)a.prev_rho + i, pr);
+    if (a.prev_u) {
+      const R* pu = (const R*)a.prev_u + i;
+      load4(pu, px);
+      load4(pu + a.N, py);
+      load4(pu + 2 * (size_t)a.N, pz);
+    }
+    if (a.phase) load4((const R*)a.phase + i, ph);
+  }
+};
+
 // Role loops over plane z: lane t of the pair takes cells (VEC: 4-cell
 // groups) t, t + stride, ... of the plane.
 template <typename R, bool VEC>
@@ -385,20 +405,38 @@ __device__ inline void stats_role_b(const StatsArgs& a, uint32_t z, uint32_t t0,
     for (uint32_t j = t0; j < a.nxy / 4; j += stride) {
       Group4<R> g;
       g.load(rho, ux_p, uy_p, uz_p, flp, j, fluid_word);
+      Extra4<R> e;
+      if constexpr (EXTRA) e.load(a, base + 4 * (size_t)j);
       const uint32_t y0 = fdiv(4 * j, a.dnx), x0 = 4 * j - y0 * a.nx;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const bool wrap = x0 + k >= a.nx;
         const uint32_t x = wrap ? x0 + k - a.nx : x0 + k, y = wrap ? y0 + 1 : y0;
         const bool in_box = zin && x - 1u < nx2 && y - 1u < ny2;
-        acc.template add<R>(a, base, 4 * j + k, in_box, g.r[k], g.x[k], g.y[k], g.w[k], g.f[k]);
+        if constexpr (EXTRA)
+          acc.template add<R>(a, in_box, g.r[k], g.x[k], g.y[k], g.w[k], g.f[k], e.pr[k], e.px[k], e.py[k], e.pz[k],
+                              e.ph[k]);
+        else
+          acc.template add<R>(a, in_box, g.r[k], g.x[k], g.y[k], g.w[k], g.f[k], R(0), R(0), R(0), R(0), R(0));
       }
     }
   } else {
     for (uint32_t i = t0; i < a.nxy; i += stride) {
       const uint32_t y = fdiv(i, a.dnx), x = i - y * a.nx;
       const bool in_box = zin && x - 1u < nx2 && y - 1u < ny2;
-      acc.template add<R>(a, base, i, in_box, rho[i], ux_p[i], uy_p[i], uz_p[i], flp ? flp[i] : fluid_word);
+      R pr = R(0), px = R(0), py = R(0), pz = R(0), ph = R(0);
+      if constexpr (EXTRA) {
+        const size_t c = base + i;
+        if (a.prev_rho) pr = ((const R*)a.prev_rho)[c];
+        if (a.prev_u) {
+          const R* pu = (const R*)a.prev_u + c;
+          px = pu[0];
+          py = pu[a.N];
+          pz = pu[2 * (size_t)a.N];
+        }
+        if (a.phase) ph = ((const R*)a.phase)[c];
+      }
+      acc.template add<R>(a, in_box, rho[i], ux_p[i], uy_p[i], uz_p[i], flp ? flp[i] : fluid_word, pr, px, py, pz, ph);
     }
   }
   acc.reduce(sh, wid, lane);
@@ -592,8 +630,9 @@ hipError_t launch_field_stats(bool real_double, const StatsArgs& s, double* out_
   const dim3 grid(s.tiles, s.nz);
   // 16-byte loads need every plane (and so every u component) to start on a
   // 4-cell boundary; nx >= 4 keeps a 4-cell group within two rows
-  const bool vec = s.nxy % 4 == 0 && s.nx >= 4;
+  auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   const bool extra = s.prev_rho || s.prev_u || s.phase;
+  const bool vec = s.nxy % 4 == 0 && s.nx >= 4 && aligned(s.prev_rho) && aligned(s.prev_u) && aligned(s.phase);
   if (real_double) {
     if (vec) launch_stats<double, true>(extra, grid, s, st);
     else launch_stats<double, false>(extra, grid, s, st);
