@@ -57,6 +57,7 @@ struct LesFdArgs {
   void* nu;               // real [N] out
   uint32_t nx, ny, nz, nxy, N;
   FastDiv dnx, dny;
+  BlockOrder ord;
   float cs2;              // (C_s * 1)^2, rounded once from double
   float nu_max;
 };
@@ -124,6 +125,7 @@ struct MultiphaseArgs {
   float* sforce;
   uint32_t nx, ny, nz, nxy, N;
   FastDiv dnx, dny;
+  BlockOrder ord;        // of k_mp_phase
   float sigma, mobility, dt, kappa, rho_air, drho;
   uint32_t apply;
 };
@@ -179,6 +181,7 @@ struct ThermalArgs {
   float omega_f;
   double omega_d;
   uint32_t conv;
+  BlockOrder ord;    // of k_thermal_collide
   uint32_t* bad;     // cells that fail the stability test of the last step
 };
 // nsteps steps ping-ponging g[gcur] / T[tcur]; base supplies the fields.

@@ -211,6 +211,36 @@ inline uint32_t launch_blocks(uint32_t order, const Grid& g) {
   return (g.nblk + S - 1) / S * S;
 }
 
+// Block order of a dense one-thread-per-cell pass that reads the neighbours in
+// z (the phase step, the finite-difference eddy viscosity, the thermal
+// convection).  Dealt round-robin, a plane's blocks leave its lines in all
+// eight L2s and the planes above and below are fetched again by other XCDs.
+// A pass whose fields stay in the last-level cache gives each XCD one range
+// of planes; one that streams from HBM keeps one front, in groups of 16
+// blocks (4096 cells) per XCD.  Measured, linear / ranges / groups of 16 (us):
+//                           phase step            eddy viscosity        convection step
+//   64^3                    7.8 / 8.0 / 7.7       6.9 / 7.0 / 6.8       8.6 / 10.3 / 10.6
+//   128^3                   14.9 / 12.9 / 14.5    14.0 / 11.2 / 12.5    39.0 / 37.2 / 38.1
+//   160^3                   28.6 / 21.7 / 27.9    28.5 / 19.9 / 27.2    76.7 / 73.9 / 74.8
+//   224^3                   80.1 / 85.8 / 75.4    82.8 / 64.1 / 63.8    228.9 / 236.6 / 222.2
+// (The pressure drive over the cup is 15-25 % slower in ranges, whose cells
+// are unevenly solid, and within 4 % in groups: it stays linear, as do passes
+// without neighbours.)
+struct BlockOrder {
+  uint32_t order, per_xcd, nblk;
+};
+inline BlockOrder linear_order(uint64_t cells) {
+  const Grid g = make_grid(cells);
+  return BlockOrder{ORDER_LINEAR, g.per_xcd, g.nblk};
+}
+// bytes: what the pass reads and writes
+inline BlockOrder stencil_order(uint64_t cells, uint64_t bytes) {
+  const Grid g = make_grid(cells);
+  return BlockOrder{bytes <= (256ull << 20) ? ORDER_XCD_RANGES : 4u, g.per_xcd, g.nblk};
+}
+inline uint32_t launch_blocks(const BlockOrder& o) { return launch_blocks(o.order, Grid{o.nblk, o.per_xcd, o.per_xcd * NXCD}); }
+__device__ inline uint32_t ordered_block(const BlockOrder& o) { return ordered_block(o.order, o.per_xcd); }
+
 // Plane-major buffer addressing.  Addr<true> keeps the element index
 // q*N + i and its byte offset in 32 bits, so an access is one 64-bit SGPR base
 // plus one 32-bit VGPR offset (global saddr form) instead of a 64-bit VGPR

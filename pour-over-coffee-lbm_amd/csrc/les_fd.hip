@@ -18,7 +18,9 @@ namespace pol {
 template <typename R>
 __global__ void __launch_bounds__(256) k_les_fd(const LesFdArgs a) {
 #pragma clang fp contract(off)
-  const uint32_t c = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t lblk = ordered_block(a.ord);
+  if (lblk >= a.ord.nblk) return;
+  const uint32_t c = lblk * 256u + threadIdx.x;
   if (c >= a.N) return;
   const uint32_t yz = fdiv(c, a.dnx);
   const uint32_t x = c - yz * a.nx;
@@ -56,8 +58,11 @@ __global__ void __launch_bounds__(256) k_les_fd(const LesFdArgs a) {
   nu[c] = v;
 }
 
-hipError_t launch_les_fd(bool dbl, const LesFdArgs& a, hipStream_t s) {
-  const dim3 grid((a.N + 255) / 256), block(256);
+hipError_t launch_les_fd(bool dbl, const LesFdArgs& a0, hipStream_t s) {
+  LesFdArgs a = a0;
+  // u (and the phase) read, nu written, flags
+  a.ord = stencil_order(a.N, ((dbl ? 8ull : 4ull) * (a.phase ? 5 : 4) + (a.flags ? 4 : 0)) * a.N);
+  const dim3 grid(launch_blocks(a.ord)), block(256);
   if (dbl) hipLaunchKernelGGL(k_les_fd<double>, grid, block, 0, s, a);
   else hipLaunchKernelGGL(k_les_fd<float>, grid, block, 0, s, a);
   return hipGetLastError();

@@ -134,7 +134,9 @@ __global__ void __launch_bounds__(256) k_mp_interface(const MultiphaseArgs a) {
 template <typename R>
 __global__ void __launch_bounds__(256) k_mp_phase(const MultiphaseArgs a) {
 #pragma clang fp contract(off)
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t lblk = ordered_block(a.ord);
+  if (lblk >= a.ord.nblk) return;
+  const uint32_t i = lblk * 256u + threadIdx.x;
   if (i >= a.N) return;
   uint32_t x, y, z;
   mp_decompose(a, i, x, y, z);
@@ -215,8 +217,10 @@ hipError_t launch_mp_interface(bool dbl, const MultiphaseArgs& a, bool out, hipS
   return hipGetLastError();
 }
 
-hipError_t launch_mp_phase(bool dbl, const MultiphaseArgs& a, hipStream_t s) {
-  const dim3 grid((a.N + 255) / 256);
+hipError_t launch_mp_phase(bool dbl, const MultiphaseArgs& a0, hipStream_t s) {
+  MultiphaseArgs a = a0;
+  a.ord = stencil_order(a.N, (dbl ? 52ull : 32ull) * a.N);  // phi, mu, u read; phi, rho, phase written
+  const dim3 grid(launch_blocks(a.ord));
   if (dbl) hipLaunchKernelGGL(k_mp_phase<double>, grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL(k_mp_phase<float>, grid, dim3(256), 0, s, a);
   return hipGetLastError();

@@ -61,7 +61,9 @@ __device__ inline void decompose(const ThermalArgs& a, uint32_t i, uint32_t& x, 
 template <typename R, bool CONV, bool WT = false>
 __global__ void __launch_bounds__(256) k_thermal_collide(const ThermalArgs a) {
 #pragma clang fp contract(off)
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t lblk = ordered_block(a.ord);
+  if (lblk >= a.ord.nblk) return;
+  const uint32_t i = lblk * 256u + threadIdx.x;
   if (i >= a.N) return;
   if (i == 0) *a.bad = 0u;  // counted by the temperature pass that follows
   uint32_t x, y, z;
@@ -302,19 +304,25 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
   // leaves the input state's temperature as the caller set it (it may be a
   // boundary value rather than sum g).
   const dim3 grid((base.N + 255) / 256);
+  // convection reads the temperature's neighbours (populations, T, u and the
+  // sources, 80 B a cell); pure diffusion reads only the cell's own values
+  const BlockOrder ord =
+      base.conv ? stencil_order(base.N, 20ull * sizeof(R) * base.N) : linear_order(base.N);
+  const dim3 cgrid(launch_blocks(ord));
   for (int n = 0; n < nsteps; ++n) {
     ThermalArgs a = base;
+    a.ord = ord;
     a.gin = g[gcur];
     a.gout = g[1 - gcur];
     a.T = T[tcur];
     a.Tout = T[1 - tcur];
     const bool last = n + 1 == nsteps;
     if (a.conv)
-      hipLaunchKernelGGL((k_thermal_collide<R, true>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((k_thermal_collide<R, true>), cgrid, dim3(256), 0, s, a);
     else if (n == 0 || !last)
-      hipLaunchKernelGGL((k_thermal_collide<R, false>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((k_thermal_collide<R, false>), cgrid, dim3(256), 0, s, a);
     else
-      hipLaunchKernelGGL((k_thermal_collide<R, false, true>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((k_thermal_collide<R, false, true>), cgrid, dim3(256), 0, s, a);
     if (a.conv || last) hipLaunchKernelGGL(k_thermal_temperature<R>, grid, dim3(256), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -11,7 +11,7 @@ from pourover_amd.thermal import ThermalFluidCoupledSolver, ThermalLBM
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(2, 2, 2), (7, 5, 3), (64, 2, 2), (33, 31, 2), (16, 17, 19), (65, 40, 21)]
+SHAPES = [(2, 2, 2), (7, 5, 3), (64, 2, 2), (33, 31, 2), (16, 17, 19), (65, 40, 21), (70, 66, 60)]
 
 
 def _make(shape, precision, convection, seed=3):
