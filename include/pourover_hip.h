@@ -545,6 +545,12 @@ int pol_thermal_init(pol_ctx *ctx, void *stream);
  * NaN, a population NaN or |g| > 1000) is copied to *unstable_out (count of
  * failing cells); synchronous then. */
 int pol_thermal_step(pol_ctx *ctx, int nsteps, int32_t *unstable_out, void *stream);
+/* As pol_thermal_step with nsteps >= 1 and convection on, after copying
+ * velocity (real [3][cells]) into the bound velocity buffer: the first step
+ * reads it from there and stores it (the coupled loop's hand-over of the fluid
+ * velocity, thermal_fluid_coupled.py:183-190, without a pass of its own).  The
+ * bound velocity buffer is written. */
+int pol_thermal_step_with_velocity(pol_ctx *ctx, int nsteps, const void *velocity, int32_t *unstable_out, void *stream);
 /* Heat flux q = -k grad T (central differences, interior cells; 0 on the
  * faces) of the current temperature into flux (real [3][cells];
  * thermal_lbm.py:268-286). */

@@ -1155,7 +1155,7 @@ static ThermalArgs thermal_args(const pol_ctx* c) {
   a.Tout = c->tb.temperature[c->tcur];
   a.hs = c->tb.heat_source;
   a.hsb = (c->td.options & POL_THERMAL_RESET_SOURCE) ? c->tb.heat_source_base : nullptr;
-  a.u = c->tb.velocity;
+  a.u = (void*)c->tb.velocity;
   a.k = c->tb.conductivity;
   a.nx = d.nx;
   a.ny = d.ny;
@@ -1219,13 +1219,13 @@ int pol_thermal_init(pol_ctx* c, void* stream) {
   return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_thermal_init");
 }
 
-int pol_thermal_step(pol_ctx* c, int nsteps, int32_t* unstable_out, void* stream) {
-  if (!c || nsteps < 0) return POL_ERR_INVALID;
-  if (!c->thermal) return fail(c, POL_ERR_STATE, "pol_thermal_step: thermal buffers not bound");
+static int thermal_step(pol_ctx* c, int nsteps, const void* velocity, int32_t* unstable_out, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipSetDevice(c->d.device);
+  ThermalArgs a = thermal_args(c);
+  a.u_src = velocity;
   if (e == hipSuccess)
-    e = launch_thermal_steps(c->d.storage == POL_F64, thermal_args(c), c->tb.g, c->tb.temperature, c->gcur, c->tcur,
+    e = launch_thermal_steps(c->d.storage == POL_F64, a, c->tb.g, c->tb.temperature, c->gcur, c->tcur,
                              nsteps, s);
   if (e == hipSuccess && unstable_out) {
     if (nsteps == 0) {
@@ -1238,6 +1238,20 @@ int pol_thermal_step(pol_ctx* c, int nsteps, int32_t* unstable_out, void* stream
     }
   }
   return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_thermal_step");
+}
+
+int pol_thermal_step(pol_ctx* c, int nsteps, int32_t* unstable_out, void* stream) {
+  if (!c || nsteps < 0) return POL_ERR_INVALID;
+  if (!c->thermal) return fail(c, POL_ERR_STATE, "pol_thermal_step: thermal buffers not bound");
+  return thermal_step(c, nsteps, nullptr, unstable_out, stream);
+}
+
+int pol_thermal_step_with_velocity(pol_ctx* c, int nsteps, const void* velocity, int32_t* unstable_out, void* stream) {
+  if (!c || !velocity || nsteps < 1) return POL_ERR_INVALID;
+  if (!c->thermal) return fail(c, POL_ERR_STATE, "pol_thermal_step_with_velocity: thermal buffers not bound");
+  if (!(c->td.options & POL_THERMAL_CONVECTION))
+    return fail(c, POL_ERR_STATE, "pol_thermal_step_with_velocity: needs POL_THERMAL_CONVECTION");
+  return thermal_step(c, nsteps, velocity, unstable_out, stream);
 }
 
 int pol_thermal_heat_flux(pol_ctx* c, void* flux, void* stream) {

@@ -174,7 +174,8 @@ struct ThermalArgs {
   void* Tout;        // temperature after the step
   void* hs;          // heat source
   const void* hsb;   // base heat source read instead of hs (reset fused), or null
-  const void* u;     // [3][N] or null
+  void* u;           // [3][N] or null
+  const void* u_src; // [3][N] velocity the first step takes over into u, or null
   const void* k;     // conductivity or null
   uint32_t nx, ny, nz, nxy, N;
   FastDiv dnx, dny;

@@ -194,11 +194,30 @@ class ThermalLBM:
     # ---- step ------------------------------------------------------------------------
     def step(self) -> bool:
         """thermal_lbm.py:396-427: True when the stability test passes."""
+        return self._step(None)
+
+    def step_with_velocity(self, velocity_field) -> bool:
+        """set_velocity_field(velocity_field) and step() in one: with
+        convection on, a device velocity of the solver's type and layout is
+        copied inside the step."""
+        src = self._velocity_source(velocity_field)
+        v = self._vel
+        if (self.is_initialized and self.enable_convection and isinstance(src, torch.Tensor) and src.device == v.device
+                and src.dtype == v.dtype and src.shape == v.shape and src.is_contiguous()):
+            return self._step(src)
+        self.set_velocity_field(src)
+        return self._step(None)
+
+    def _step(self, velocity: Optional[torch.Tensor]) -> bool:
         if not self.is_initialized:
             return False
         u = C.c_int32()
-        L.check(self.lib.pol_thermal_step(self.ctx.handle, 1, C.byref(u), L.stream_handle()), self.ctx.handle,
-                "pol_thermal_step")
+        if velocity is None:
+            st = self.lib.pol_thermal_step(self.ctx.handle, 1, C.byref(u), L.stream_handle())
+        else:
+            st = self.lib.pol_thermal_step_with_velocity(self.ctx.handle, 1, velocity.data_ptr(), C.byref(u),
+                                                         L.stream_handle())
+        L.check(st, self.ctx.handle, "pol_thermal_step")
         self._gcur ^= 1
         self._tcur ^= 1
         self._last_unstable = int(u.value)
@@ -304,12 +323,13 @@ class ThermalLBM:
         solver with `u`) into the thermal solver's velocity buffer."""
         if not self.enable_convection:
             return
-        src = velocity_field
+        self._vel.copy_(self._velocity_source(velocity_field))
+
+    @staticmethod
+    def _velocity_source(src):
         if hasattr(src, "u") and not isinstance(src, (torch.Tensor, DeviceField)):
             src = src.u
-        if isinstance(src, DeviceField):
-            src = src.to_torch()
-        self._vel.copy_(src)
+        return src.to_torch() if isinstance(src, DeviceField) else src
 
     def use_base_heat_source(self, base_heat_source, enable: bool = True) -> None:
         """Start every following step from base_heat_source (the coupled
@@ -409,15 +429,19 @@ class ThermalFluidCoupledSolver:
         self.fluid_solver.step()
         t1 = time.time()
         self.performance_stats["fluid_time"] += t1 - t0
+        velocity = None  # handed over inside the first sub-cycle
         if self.coupling_step % cfg.coupling_frequency == 0:
             get = getattr(self.fluid_solver, "get_velocity_field_for_thermal_coupling", None)
-            self.thermal_solver.set_velocity_field(get() if get is not None else self.fluid_solver.u)
+            velocity = get() if get is not None else self.fluid_solver.u
+            if cfg.thermal_subcycles < 1:
+                self.thermal_solver.set_velocity_field(velocity)
             self.performance_stats["coupling_time"] += time.time() - t1
         t2 = time.time()
         if not self.fused_reset:
             self.thermal_solver.reset_heat_source_to_base(self.base_heat_source)
-        for _ in range(cfg.thermal_subcycles):
-            if not self.thermal_solver.step():
+        for k in range(cfg.thermal_subcycles):
+            hand_over = k == 0 and velocity is not None
+            if not (self.thermal_solver.step_with_velocity(velocity) if hand_over else self.thermal_solver.step()):
                 return False
         self.performance_stats["thermal_time"] += time.time() - t2
         if cfg.enable_diagnostics and not self._check_coupling_stability():

@@ -47,6 +47,26 @@ def test_run_equals_single_steps(shape, precision, convection):
 
 
 @pytest.mark.parametrize("precision", ["f32", "f64"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_step_with_velocity(shape, precision):
+    """The velocity handed over inside the step: the state and the velocity
+    buffer of set_velocity_field and step, for a device velocity, one that
+    needs a conversion or a copy, and the solver's own buffer."""
+    rng = np.random.default_rng(11)
+    a, b = _make(shape, precision, True), _make(shape, precision, True)
+    other = torch.float64 if precision == "f32" else torch.float32
+    for kind in ("same", "type", "strided", "own", "host"):
+        u = torch.from_numpy(rng.uniform(-0.02, 0.02, tuple(a._vel.shape))).to(a._vel)
+        u = {"same": u, "type": u.to(other), "strided": u.flip(0).transpose(1, 3).contiguous().transpose(1, 3),
+             "own": None, "host": u.cpu()}[kind]
+        ok = a.step_with_velocity(a._vel if u is None else u)
+        b.set_velocity_field(b._vel if u is None else u)
+        assert ok == b.step()
+        for x, y in ((a._vel, b._vel), (a.g_device, b.g_device), (a._hs, b._hs), (a._T[a._tcur], b._T[b._tcur])):
+            assert torch.equal(x, y), kind
+
+
+@pytest.mark.parametrize("precision", ["f32", "f64"])
 @pytest.mark.parametrize("shape", SHAPES + [(128, 64, 33), (101, 103, 107)])
 def test_statistics(shape, precision):
     print("case: thermal statistics %s %s" % (shape, precision), flush=True)
