@@ -416,6 +416,14 @@ int pol_adjoint_sweep(pol_ctx *ctx, const void *states, uint64_t stride_bytes, i
  * forward states from the first (the checkpointed reverse sweep; no
  * counterpart in the reference). */
 int pol_step_chain(pol_ctx *ctx, void *states, uint64_t stride_bytes, int count, void *stream);
+/* count >= 1 fused steps in one call, step i from states + i * stride_bytes
+ * into states + (i + 1) * stride_bytes and the last into final_state: records
+ * the forward states of the adjoint.  The steps i >= flux_first also give
+ * their outlet mass flux (POL_RED_OUTFLUX, FP64) in flux_out[i - flux_first]
+ * (host; NULL when flux_first >= count); with any, the call waits for the
+ * stream once, at the end (and every 43 + nz fluxes). */
+int pol_step_record(pol_ctx *ctx, void *states, uint64_t stride_bytes, int count, void *final_state, int flux_first,
+                    double *flux_out, void *stream);
 /* Zero the adjoint state, grad_perm and the inlet-velocity gradient. */
 int pol_adjoint_reset(pol_ctx *ctx, void *stream);
 /* Fold and copy the FP64 accumulators {dJ/du_in x, y, z, J} (4 doubles) to

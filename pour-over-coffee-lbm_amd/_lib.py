@@ -218,6 +218,7 @@ SIGNATURES = {
     "pol_adjoint_reset": (C.c_int, [_P, _P]),
     "pol_adjoint_sweep": (C.c_int, [_P, _P, C.c_uint64, C.c_int, C.c_int, _P]),
     "pol_step_chain": (C.c_int, [_P, _P, C.c_uint64, C.c_int, _P]),
+    "pol_step_record": (C.c_int, [_P, _P, C.c_uint64, C.c_int, _P, C.c_int, _P, _P]),
     "pol_adjoint_collect": (C.c_int, [_P, _P, _P]),
     "pol_field_stats": (C.c_int, [_P, C.POINTER(PolStatsOpts), _P, _P, _P]),
     "pol_export_fields": (C.c_int, [_P, _P, _P, _P]),

@@ -115,14 +115,8 @@ class AdjointProblem:
         J = 0.0
         self._seg_holds = None
         if checkpoints and self.store_all:
-            seg = self.seg
-            seg[0].copy_(ctx.f_current)
-            for n in range(self.steps):
-                out = seg[n + 1] if n + 1 < self.steps else ctx.f_next
-                what = L.POL_WANT_REDUCE if self.objective_step(n) else 0
-                red = ctx.step_from(seg[n], out, what)
-                if what:
-                    J += float(red[7])
+            self.seg[0].copy_(ctx.f_current)
+            J = self._record(0)
             ctx.set_current(1 - ctx.current)  # the final state is the context's current one
             return J
         K = self.checkpoint
@@ -130,28 +124,33 @@ class AdjointProblem:
         for n in range(self.steps):
             if checkpoints and n % K == 0:
                 self.ckpt[n // K].copy_(ctx.f_current)
-            if checkpoints and n >= last:
+            if checkpoints and n == last:
                 # f^n .. f^{steps-1} into the segment store, the final state
                 # into the context's next buffer (the same fused step as
                 # ctx.step, from and into other buffers)
-                seg = self.seg
-                if n == last:
-                    seg[0].copy_(ctx.f_current)
-                out = seg[n - last + 1] if n + 1 < self.steps else ctx.f_next
-                what = L.POL_WANT_REDUCE if self.objective_step(n) else 0
-                red = ctx.step_from(seg[n - last], out, what)
-                if what:
-                    J += float(red[7])
-                if n + 1 == self.steps:
-                    self._seg_holds = self.steps // K - 1
-                    ctx.set_current(1 - ctx.current)  # the final state is the context's current one
-                continue
+                self.seg[0].copy_(ctx.f_current)
+                J += self._record(last)
+                self._seg_holds = self.steps // K - 1
+                ctx.set_current(1 - ctx.current)  # the final state is the context's current one
+                break
             if self.objective_step(n):
                 red = ctx.step(1, L.POL_WANT_REDUCE)
                 J += float(red[7])
             else:
                 ctx.step(1)
         return J
+
+    def _record(self, start: int) -> float:
+        """Steps start .. start + checkpoint - 1 from seg[0] through the segment
+        store, the last into the context's next buffer, in one native call;
+        the sum of their objective steps' outlet fluxes."""
+        ctx, K = self.ctx, self.checkpoint
+        first = max(0, min(K, (self.steps - self.window) - start))  # first objective step of these
+        flux = np.zeros(max(K - first, 1), dtype=np.float64)
+        stride = self.seg[0].numel() * self.seg.element_size()
+        L.check(ctx.lib.pol_step_record(ctx.handle, L.ptr(self.seg), stride, K, L.ptr(ctx.f_next), first,
+                                        flux.ctypes.data, L.stream_handle()), ctx.handle, "pol_step_record")
+        return sum(flux.tolist(), 0.0)
 
     def forward_time(self) -> float:
         """Seconds for the plain forward run (no reductions, no checkpoints)."""

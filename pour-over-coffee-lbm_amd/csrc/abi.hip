@@ -26,6 +26,7 @@ struct pol_ctx {
   double* partial = nullptr;  // [nblk][POL_NRED]
   uint32_t* bad_dev = nullptr;  // [1] cells failing the thermal stability test
   double* host = nullptr;     // pinned [POL_NSTAT + nz]: results on their way to the caller
+  int host_cap() const { return POL_NSTAT + d.nz; }
   // particles
   bool particles = false;
   bool pcoupled = false;  // the implicit drag field holds the footprint of a coupling
@@ -35,7 +36,6 @@ struct pol_ctx {
   pol_adjoint_buffers ab{};
   int acur = 0;
   double* adj_partial = nullptr;  // [nblk][4]
-  double* adj_acc = nullptr;      // [4]: dJ/du_in (3), J
   // field statistics
   uint32_t stat_tiles = 0;          // blocks per z plane
   double* stat_partial = nullptr;   // [nz * stat_tiles][POL_NSTAT]
@@ -136,7 +136,6 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
   if (e == hipSuccess) e = hipMalloc((void**)&c->partial, (size_t)c->part_cap * POL_NRED * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&c->bad_dev, sizeof(uint32_t));
   if (e == hipSuccess) e = hipMalloc((void**)&c->adj_partial, (size_t)c->part_cap * 4 * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void**)&c->adj_acc, 4 * sizeof(double));
   // statistics: up to 12 blocks per plane (2688 blocks at 224^3, each lane
   // ~8 groups of four cells: the per-block reduction of the 43 statistics is
   // amortised; 224^3 V60 kernel 0.062 ms against 0.069 / 0.067 ms with 8 / 24)
@@ -155,7 +154,6 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
     (void)hipFree(c->partial);
     (void)hipFree(c->bad_dev);
     (void)hipFree(c->adj_partial);
-    (void)hipFree(c->adj_acc);
     (void)hipFree(c->stat_partial);
     (void)hipFree(c->stat_zpart);
     (void)hipFree(c->stat_dev);
@@ -172,7 +170,6 @@ int pol_destroy(pol_ctx* c) {
   (void)hipFree(c->partial);
   (void)hipFree(c->bad_dev);
   (void)hipFree(c->adj_partial);
-  (void)hipFree(c->adj_acc);
   (void)hipFree(c->stat_partial);
   (void)hipFree(c->stat_zpart);
   (void)hipFree(c->stat_dev);
@@ -765,7 +762,6 @@ int pol_adjoint_reset(pol_ctx* c, void* stream) {
   if (e == hipSuccess) e = hipMemsetAsync(c->ab.lam[1], 0, (size_t)POL_Q * c->P * rb, s);
   if (e == hipSuccess && c->ab.grad_perm) e = hipMemsetAsync(c->ab.grad_perm, 0, (size_t)c->N * sizeof(double), s);
   if (e == hipSuccess) e = hipMemsetAsync(c->adj_partial, 0, (size_t)c->wgrid.nblk * 4 * sizeof(double), s);
-  if (e == hipSuccess) e = hipMemsetAsync(c->adj_acc, 0, 4 * sizeof(double), s);
   c->acur = 0;
   return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_adjoint_reset");
 }
@@ -819,15 +815,43 @@ int pol_step_chain(pol_ctx* c, void* states, uint64_t stride_bytes, int count, v
   return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_step_chain");
 }
 
+int pol_step_record(pol_ctx* c, void* states, uint64_t stride_bytes, int count, void* final_state, int flux_first,
+                    double* flux_out, void* stream) {
+  if (!c || !states || !final_state || count < 1 || flux_first < 0) return POL_ERR_INVALID;
+  if (!c->bound) return fail(c, POL_ERR_STATE, "pol_step_record: buffers not bound");
+  if (les_fd(c)) return fail(c, POL_ERR_UNSUPPORTED, "pol_step_record: not with the finite-difference LES");
+  if (count > 1 && stride_bytes == 0) return fail(c, POL_ERR_INVALID, "pol_step_record: zero state stride");
+  if (flux_first < count && !flux_out) return fail(c, POL_ERR_INVALID, "pol_step_record: flux_out is NULL");
+  hipStream_t s = (hipStream_t)stream;
+  hipError_t e = hipSetDevice(c->d.device);
+  int held = 0;  // fluxes in the pinned buffer
+  for (int i = 0; i < count && e == hipSuccess; ++i) {
+    const bool flux = i >= flux_first;
+    const StepArgs a = make_args(c, (const char*)states + (uint64_t)i * stride_bytes,
+                                 i + 1 < count ? (char*)states + (uint64_t)(i + 1) * stride_bytes : final_state,
+                                 flux ? WANT_FLUX : 0u);
+    e = launch_stream_collide(c->d.storage, a, true, c->wgrid, s);
+    if (e != hipSuccess || !flux) continue;
+    e = launch_flux_fold(c->partial, c->wgrid.nblk, c->host + held++, s);
+    if (e == hipSuccess && (held == c->host_cap() || i + 1 == count)) {
+      e = hipStreamSynchronize(s);
+      if (e == hipSuccess) std::memcpy(flux_out + (i + 1 - flux_first - held), c->host, held * sizeof(double));
+      held = 0;
+    }
+  }
+  return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_step_record");
+}
+
 int pol_adjoint_collect(pol_ctx* c, double* out4, void* stream) {
   if (!c || !out4) return POL_ERR_INVALID;
   if (!c->adjoint) return fail(c, POL_ERR_STATE, "pol_adjoint_collect: adjoint not bound");
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipSetDevice(c->d.device);
-  if (e == hipSuccess) e = launch_adjoint_final(c->adj_partial, c->wgrid.nblk, c->adj_acc, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(out4, c->adj_acc, 4 * sizeof(double), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = launch_adjoint_final(c->adj_partial, c->wgrid.nblk, c->host, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_adjoint_collect");
+  if (e != hipSuccess) return hip_fail(c, e, "pol_adjoint_collect");
+  std::memcpy(out4, c->host, 4 * sizeof(double));
+  return POL_OK;
 }
 
 // ---- field diagnostics --------------------------------------------------------

@@ -63,6 +63,12 @@ struct LesFdArgs {
 };
 hipError_t launch_les_fd(bool dbl, const LesFdArgs& a, hipStream_t s);
 
+// StepArgs::what bit beside POL_WANT_*: the step's outlet mass flux
+// (POL_RED_OUTFLUX) per block into partial[block].
+constexpr uint32_t WANT_FLUX = 0x80000000u;
+// Fold those partials into out[0] (device or pinned host memory), in a fixed order.
+hipError_t launch_flux_fold(const double* partial, uint32_t nblk, double* out, hipStream_t s);
+
 // Launch one pass.  store_f: write post-collision populations (a step);
 // false = moments only (macro/reduce of the current state).
 hipError_t launch_stream_collide(int storage, const StepArgs& a, bool store_f, const Grid& g, hipStream_t s);

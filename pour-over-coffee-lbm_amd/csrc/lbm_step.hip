@@ -51,6 +51,20 @@ __global__ void __launch_bounds__(256) k_reduce_fold(double* partial, uint32_t r
   }
 }
 
+// One double per block (2 669 at 128^3, 14 784 at 224^3): latency bound, so the
+// lanes keep eight loads in flight.
+__global__ void __launch_bounds__(256) k_flux_fold(const double* __restrict__ partial, uint32_t nblk,
+                                                   double* __restrict__ out) {
+  double v = 0.0;
+#pragma unroll 8
+  for (uint32_t b = threadIdx.x; b < nblk; b += 256) v += partial[b];
+  v = wave_sum(v);
+  __shared__ double sh[4];
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) out[0] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
 template <typename S>
 __global__ void __launch_bounds__(256) k_init_equilibrium(S* __restrict__ f, const typename Codec<S>::real* rho,
                                                           const typename Codec<S>::real* u, uint32_t N) {
@@ -207,6 +221,11 @@ hipError_t launch_reduce_final(double* partial, uint32_t nblk, double* out, hipS
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(k_reduce_fold, dim3(1), dim3(256), 0, s, partial, rows, stride, rows, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_flux_fold(const double* partial, uint32_t nblk, double* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_flux_fold, dim3(1), dim3(256), 0, s, partial, nblk, out);
   return hipGetLastError();
 }
 

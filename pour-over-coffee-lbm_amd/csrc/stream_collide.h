@@ -227,6 +227,17 @@ __global__ void __launch_bounds__(BLOCK) k_stream_collide(const StepArgs a) {
       u[2 * (size_t)N + cell] = o.uz;
     }
   }
+  if (a.what & WANT_FLUX) {
+    // the step's outlet mass flux alone (the adjoint's objective): few waves
+    // hold outlet cells, the others only meet the barrier
+    __shared__ double shf[BLOCK / 64];
+    const bool out = active && kind == POL_KIND_OUTLET;
+    double r = 0.0;
+    if (__ballot(out) != 0ull) r = wave_sum(out ? -(1.0 + (double)o.rd) * (double)o.uz : 0.0);
+    if ((threadIdx.x & 63) == 0) shf[threadIdx.x >> 6] = r;
+    __syncthreads();
+    if (threadIdx.x == 0) a.partial[lblk] = (shf[0] + shf[1]) + (shf[2] + shf[3]);
+  }
   if (a.what & POL_WANT_REDUCE) {
     double v[POL_NRED];
 #pragma unroll
