@@ -289,10 +289,20 @@ def check(status: int, ctx=None, what: str = "") -> None:
     raise PolError(status, "%s failed: %s%s" % (what or "pol call", base, (" - " + detail) if detail else ""))
 
 
+# torch's raw current-stream query: 0.1 us, where torch.cuda.current_stream()
+# takes 2.9 us to build a Stream object (of about 7 us for a whole call of a
+# launch entry point).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def stream_handle(stream=None):
-    """hipStream_t of a torch stream (default: current stream)."""
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return C.c_void_p(s.cuda_stream)
+    """hipStream_t of a torch stream (default: the current device's current stream)."""
+    if stream is None:
+        if _raw_stream is not None and _raw_device is not None and torch.cuda.is_initialized():
+            return C.c_void_p(_raw_stream(_raw_device()))
+        stream = torch.cuda.current_stream()
+    return C.c_void_p(stream.cuda_stream)
 
 
 def ptr(t) -> C.c_void_p:
