@@ -304,14 +304,24 @@ static StepArgs make_args(const pol_ctx* c, const void* fin, void* fout, uint32_
   // Streaming (non-temporal) stores once a step's population traffic (read +
   // write) exceeds the 256 MiB last-level cache: at 224^3 they cut the V60
   // step by 7 % (FP32 compact), 13 % (FP16) and 8 % (FP64); at 128^3, where
-  // the step still caches, they cost 25 %.
-  a.stream_store = 2ull * a.n_items * Q * storage_bytes(d.storage) > (256ull << 20) ? 1u : 0u;
+  // the step still caches, they cost 25 %.  Not where the planes of an
+  // unlisted dense box are no whole number of 64-byte sectors apart: a wave's
+  // stores then end inside sectors, which streaming sends to HBM as
+  // read-modify-writes, while cached stores of neighbouring blocks meet in
+  // one L2 (FP32 180 x 175 x 179: 228 -> 174 us, 241 x 239 x 243: 573 -> 422,
+  // FP16 187 x 150 x 201: 125 -> 101; planes 64 or 128 bytes off a 256-byte
+  // boundary are up to 5 % faster streamed).
+  const bool streams = 2ull * a.n_items * Q * storage_bytes(d.storage) > (256ull << 20);
+  const bool whole_sectors = a.chunks || ((uint64_t)c->P * storage_bytes(d.storage)) % 64 == 0;
+  a.stream_store = streams && whole_sectors ? 1u : 0u;
   // Streaming steps sweep one memory front: linear blocks over the dense
-  // grid, groups of 4 consecutive blocks per XCD over the compact chunk list.
+  // grid, groups of 4 consecutive blocks per XCD over the compact chunk list,
+  // groups of 32 where split sectors have to meet in an L2 (the sizes above,
+  // linear / 4 / 32: 194 / 179 / 174, - / 434 / 422, 118 / 105 / 101 us).
   // A step that stays in the last-level cache keeps each XCD on one
   // contiguous range, whose neighbour rows then hit its own L2 (128^3 V60
   // FP32: 0.0203 ms against 0.0223 ms linear).
-  a.order = a.stream_store ? (a.records ? 2u : ORDER_LINEAR) : ORDER_XCD_RANGES;
+  a.order = !streams ? ORDER_XCD_RANGES : (a.records ? 2u : (whole_sectors ? ORDER_LINEAR : 5u));
   a.per_xcd = c->wgrid.per_xcd;
   a.nblk = c->wgrid.nblk;
   a.options = d.options;
