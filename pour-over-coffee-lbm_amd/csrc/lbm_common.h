@@ -226,6 +226,7 @@ inline uint32_t launch_blocks(uint32_t order, const Grid& g) {
 // (The pressure drive over the cup is 15-25 % slower in ranges, whose cells
 // are unevenly solid, and within 4 % in groups: it stays linear, as do passes
 // without neighbours.)
+constexpr uint64_t LAST_LEVEL_BYTES = 256ull << 20;
 struct BlockOrder {
   uint32_t order, per_xcd, nblk;
 };
@@ -236,10 +237,17 @@ inline BlockOrder linear_order(uint64_t cells) {
 // bytes: what the pass reads and writes
 inline BlockOrder stencil_order(uint64_t cells, uint64_t bytes) {
   const Grid g = make_grid(cells);
-  return BlockOrder{bytes <= (256ull << 20) ? ORDER_XCD_RANGES : 4u, g.per_xcd, g.nblk};
+  return BlockOrder{bytes <= LAST_LEVEL_BYTES ? ORDER_XCD_RANGES : 4u, g.per_xcd, g.nblk};
 }
 inline uint32_t launch_blocks(const BlockOrder& o) { return launch_blocks(o.order, Grid{o.nblk, o.per_xcd, o.per_xcd * NXCD}); }
 __device__ inline uint32_t ordered_block(const BlockOrder& o) { return ordered_block(o.order, o.per_xcd); }
+
+// A store that leaves the caches to others (NT) or an ordinary one.
+template <bool NT, typename T>
+__device__ inline void store_as(T* p, T v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
 
 // Plane-major buffer addressing.  Addr<true> keeps the element index
 // q*N + i and its byte offset in 32 bits, so an access is one 64-bit SGPR base
