@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 import torch
 
+from oracle import thermal as OT
 from pourover_amd.thermal import ThermalFluidCoupledSolver, ThermalLBM
 
 pytestmark = pytest.mark.gpu
@@ -111,3 +112,22 @@ def test_count_of_unstable_cells(shape):
 
 class _Fluid:
     """The coupled solver asks its fluid solver for nothing in these checks."""
+
+
+@pytest.mark.parametrize("convection", [False, True])
+@pytest.mark.parametrize("precision,shape", [("f32", (171, 168, 173)), ("f64", (131, 130, 145))])
+def test_streaming_steps(precision, shape, convection):
+    """Population buffers above the last-level cache (stores past the cache):
+    three steps in one run and one by one against the numpy restatement."""
+    print("case: streaming thermal steps %s %s convection=%s" % (shape, precision, convection), flush=True)
+    a = _make(shape, precision, convection)
+    assert 2 * a.g_device.numel() * a.g_device.element_size() > 256 << 20
+    T = np.ascontiguousarray(a.temperature.to_numpy())
+    st = {"g": OT.equilibrium(T), "T": T, "heat_source": np.zeros_like(T),
+          "u": np.ascontiguousarray(a._vel.cpu().numpy().transpose(3, 2, 1, 0))}
+    assert a.run(3)
+    for _ in range(3):
+        st = OT.step(st, a.omega_thermal, convection=convection)
+    assert np.array_equal(a.g, st["g"]) and np.array_equal(a.temperature.to_numpy(), st["T"])
+    assert np.array_equal(a.temperature_old.to_numpy(), st["T_old"])
+    assert np.array_equal(a.heat_source.to_numpy(), st["heat_source"])
