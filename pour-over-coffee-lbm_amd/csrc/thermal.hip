@@ -248,22 +248,36 @@ __global__ void __launch_bounds__(256) k_thermal_stats(const R* __restrict__ T, 
   }
 }
 
-// Fold of at most STAT_BLOCKS rows {min, max, sum, count} into out (pinned host memory)
+// Fold of at most STAT_BLOCKS rows {min, max, sum, count} into out (pinned host
+// memory): four rows of loads in flight per lane, then across the lanes that
+// hold the same column.
 __global__ void __launch_bounds__(256) k_thermal_fold(const double* __restrict__ partial, uint32_t rows,
                                                       double* __restrict__ out) {
-  __shared__ double sh[64][STAT_ROW];
+  __shared__ double sh[4][STAT_ROW];
   const int s = threadIdx.x & 3, j = threadIdx.x >> 2;
   auto add = [&](double r, double p) { return s == 0 ? fmin(r, p) : (s == 1 ? fmax(r, p) : r + p); };
-  double v = s == 0 ? 1.0e300 : (s == 1 ? -1.0e300 : 0.0);
-#pragma unroll 8
-  for (uint32_t b = j; b < rows; b += 64) v = add(v, partial[(size_t)b * STAT_ROW + s]);
-  sh[j][s] = v;
-  __syncthreads();
-  if (threadIdx.x < STAT_ROW) {
-    double r = sh[0][threadIdx.x];
-    for (int k = 1; k < 64; ++k) r = add(r, sh[k][threadIdx.x]);
-    out[threadIdx.x] = r;
+  const double id = s == 0 ? 1.0e300 : (s == 1 ? -1.0e300 : 0.0);
+  double v = id;
+  for (uint32_t b = j; b < rows; b += 256) {
+    double t[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) t[k] = b + 64 * k < rows ? partial[(size_t)(b + 64 * k) * STAT_ROW + s] : id;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v = add(v, t[k]);
   }
+  double x, y;
+  lane_pair<32>(v, x, y);
+  v = add(x, y);
+  lane_pair<16>(v, x, y);
+  v = add(x, y);
+  lane_pair<8>(v, x, y);
+  v = add(x, y);
+  lane_pair<4>(v, x, y);
+  v = add(x, y);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane < STAT_ROW) sh[wid][lane] = v;
+  __syncthreads();
+  if (threadIdx.x < STAT_ROW) out[threadIdx.x] = add(add(sh[0][s], sh[1][s]), add(sh[2][s], sh[3][s]));
 }
 
 template <typename R>
