@@ -557,8 +557,11 @@ int pol_thermal_step(pol_ctx *ctx, int nsteps, int32_t *unstable_out, void *stre
  * velocity (real [3][cells]) into the bound velocity buffer: the first step
  * reads it from there and stores it (the coupled loop's hand-over of the fluid
  * velocity, thermal_fluid_coupled.py:183-190, without a pass of its own).  The
- * bound velocity buffer is written. */
-int pol_thermal_step_with_velocity(pol_ctx *ctx, int nsteps, const void *velocity, int32_t *unstable_out, void *stream);
+ * bound velocity buffer is written.  With stats4 != NULL it receives what
+ * pol_thermal_coupling_stats would return after the steps, formed inside them;
+ * synchronous then. */
+int pol_thermal_step_with_velocity(pol_ctx *ctx, int nsteps, const void *velocity, int32_t *unstable_out,
+                                   double *stats4, void *stream);
 /* Heat flux q = -k grad T (central differences, interior cells; 0 on the
  * faces) of the current temperature into flux (real [3][cells];
  * thermal_lbm.py:268-286). */

@@ -227,7 +227,7 @@ SIGNATURES = {
     "pol_thermal_set": (C.c_int, [_P, C.POINTER(PolThermalDesc)]),
     "pol_thermal_init": (C.c_int, [_P, _P]),
     "pol_thermal_step": (C.c_int, [_P, C.c_int, _P, _P]),
-    "pol_thermal_step_with_velocity": (C.c_int, [_P, C.c_int, _P, _P, _P]),
+    "pol_thermal_step_with_velocity": (C.c_int, [_P, C.c_int, _P, _P, _P, _P]),
     "pol_thermal_heat_flux": (C.c_int, [_P, _P, _P]),
     "pol_thermal_stats": (C.c_int, [_P, _P, _P]),
     "pol_thermal_coupling_stats": (C.c_int, [_P, _P, _P]),

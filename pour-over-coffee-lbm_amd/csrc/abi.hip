@@ -24,7 +24,7 @@ struct pol_ctx {
   uint32_t P = 0;         // population plane stride (N, or the compact layout's stored cells)
   uint32_t part_cap = 0;  // blocks the partial buffers hold (any work grid fits)
   double* partial = nullptr;  // [nblk][POL_NRED]
-  uint32_t* bad_dev = nullptr;  // [1] cells failing the thermal stability test
+  uint32_t* bad_dev = nullptr;  // [2] cells failing the thermal stability test, cells with |u| > 1
   double* host = nullptr;     // pinned [POL_NSTAT + nz]: results on their way to the caller
   int host_cap() const { return POL_NSTAT + d.nz; }
   // particles
@@ -134,7 +134,9 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
   c->part_cap = make_grid((uint64_t)d.ny * d.nz * ((uint64_t)d.nx + 63)).nblk;
   hipError_t e = hipSetDevice(d.device);
   if (e == hipSuccess) e = hipMalloc((void**)&c->partial, (size_t)c->part_cap * POL_NRED * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void**)&c->bad_dev, sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMalloc((void**)&c->bad_dev, 2 * sizeof(uint32_t));
+  const uint32_t none[2] = {0u, 0u};
+  if (e == hipSuccess) e = hipMemcpy(c->bad_dev, none, sizeof(none), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc((void**)&c->adj_partial, (size_t)c->part_cap * 4 * sizeof(double));
   // statistics: up to 12 blocks per plane (2688 blocks at 224^3, each lane
   // ~8 groups of four cells: the per-block reduction of the 43 statistics is
@@ -1253,15 +1255,23 @@ int pol_thermal_init(pol_ctx* c, void* stream) {
   return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_thermal_init");
 }
 
-static int thermal_step(pol_ctx* c, int nsteps, const void* velocity, int32_t* unstable_out, void* stream) {
+static int thermal_step(pol_ctx* c, int nsteps, const void* velocity, int32_t* unstable_out, double* stats4,
+                        void* stream) {
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipSetDevice(c->d.device);
   ThermalArgs a = thermal_args(c);
   a.u_src = velocity;
+  a.report = stats4 ? 1u : 0u;
   if (e == hipSuccess)
     e = launch_thermal_steps(c->d.storage == POL_F64, a, c->tb.g, c->tb.temperature, c->gcur, c->tcur,
-                             nsteps, s);
-  if (e == hipSuccess && unstable_out) {
+                             nsteps, c->partial, c->host, s);
+  if (e == hipSuccess && stats4) {
+    e = hipStreamSynchronize(s);
+    if (e == hipSuccess) {
+      std::memcpy(stats4, c->host, 4 * sizeof(double));
+      if (unstable_out) *unstable_out = (int32_t)c->host[4];
+    }
+  } else if (e == hipSuccess && unstable_out) {
     if (nsteps == 0) {
       *unstable_out = 0;
     } else {
@@ -1277,15 +1287,16 @@ static int thermal_step(pol_ctx* c, int nsteps, const void* velocity, int32_t* u
 int pol_thermal_step(pol_ctx* c, int nsteps, int32_t* unstable_out, void* stream) {
   if (!c || nsteps < 0) return POL_ERR_INVALID;
   if (!c->thermal) return fail(c, POL_ERR_STATE, "pol_thermal_step: thermal buffers not bound");
-  return thermal_step(c, nsteps, nullptr, unstable_out, stream);
+  return thermal_step(c, nsteps, nullptr, unstable_out, nullptr, stream);
 }
 
-int pol_thermal_step_with_velocity(pol_ctx* c, int nsteps, const void* velocity, int32_t* unstable_out, void* stream) {
+int pol_thermal_step_with_velocity(pol_ctx* c, int nsteps, const void* velocity, int32_t* unstable_out, double* stats4,
+                                   void* stream) {
   if (!c || !velocity || nsteps < 1) return POL_ERR_INVALID;
   if (!c->thermal) return fail(c, POL_ERR_STATE, "pol_thermal_step_with_velocity: thermal buffers not bound");
   if (!(c->td.options & POL_THERMAL_CONVECTION))
     return fail(c, POL_ERR_STATE, "pol_thermal_step_with_velocity: needs POL_THERMAL_CONVECTION");
-  return thermal_step(c, nsteps, velocity, unstable_out, stream);
+  return thermal_step(c, nsteps, velocity, unstable_out, stats4, stream);
 }
 
 int pol_thermal_heat_flux(pol_ctx* c, void* flux, void* stream) {

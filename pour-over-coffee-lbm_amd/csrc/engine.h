@@ -189,11 +189,15 @@ struct ThermalArgs {
   double omega_d;
   uint32_t conv;
   BlockOrder ord;    // of k_thermal_collide
-  uint32_t* bad;     // cells that fail the stability test of the last step
+  uint32_t* bad;     // [2] cells that fail the stability test of the last step, cells with |u_src| > 1
+  uint32_t report;   // also the statistics of the state after the last step
 };
-// nsteps steps ping-ponging g[gcur] / T[tcur]; base supplies the fields.
+// nsteps steps ping-ponging g[gcur] / T[tcur]; base supplies the fields.  With
+// base.report (and base.u_src) the last step leaves {min, max, sum} of T, the
+// number of cells with |u_src| > 1 and the number that fail the stability test
+// in out[5] (pinned host memory); partial as for launch_thermal_stats.
 hipError_t launch_thermal_steps(bool dbl, const ThermalArgs& base, void* const g[2], void* const T[2], int& gcur,
-                                int& tcur, int nsteps, hipStream_t s);
+                                int& tcur, int nsteps, double* partial, double* out, hipStream_t s);
 // {min, max, sum} of T and, where u (real [3][N]) is not null, the number of
 // cells with |u| > 1 (else 0) into out[4] (device or pinned host memory);
 // partial holds at least 4 x min(1024, ceil(N / 256)) doubles.

@@ -41,6 +41,18 @@ __host__ __device__ constexpr R TW(int q) {
   return q == 0 ? R(0.25) : R(0.125);
 }
 
+constexpr uint32_t STAT_BLOCKS = 1024;
+constexpr int STAT_ROW = 4;
+
+// |u| > 1.  The rounded square root of s exceeds 1 exactly when s is above the
+// first value after 1 (sqrt(1 + eps) rounds to 1), so none is taken.
+template <typename R>
+__device__ inline bool faster_than_one(R x, R y, R z) {
+#pragma clang fp contract(off)
+  constexpr R after_one = R(1) + (sizeof(R) == 4 ? R(0x1p-23) : R(0x1p-52));
+  return (x * x + y * y) + z * z > after_one;
+}
+
 template <typename R>
 __device__ inline R omega_of(const ThermalArgs& a) {
   if constexpr (sizeof(R) == 4) return a.omega_f;
@@ -100,6 +112,11 @@ __global__ void __launch_bounds__(256) k_thermal_collide(const ThermalArgs a) {
     u[i] = v0;
     u[N + i] = v1;
     u[2 * N + i] = v2;
+    if (a.report) {  // cells with |u| > 1: zero on entry, taken and cleared by the fold
+      const bool fast = faster_than_one(v0, v1, v2);
+      const uint64_t cells = __ballot(fast);
+      if (fast && (cells & ((1ull << (threadIdx.x & 63)) - 1ull)) == 0ull) atomicAdd(a.bad + 1, (uint32_t)__popcll(cells));
+    }
   }
   if constexpr (CONV) {
     if (x >= 1 && x + 1 < a.nx && y >= 1 && y + 1 < a.ny && z >= 1 && z + 1 < a.nz) {
@@ -146,87 +163,8 @@ __global__ void __launch_bounds__(256) k_thermal_collide(const ThermalArgs a) {
   }
 }
 
-// T' = sum_q g'_q and the stability test.  Bound by reading the populations
-// (224^3: 0.075 ms for 360 MB).  Failing cells are counted in *a.bad, which
-// the collide pass before has set to zero: a wave without one (every wave of
-// a stable state) neither reduces nor stores anything.  A count per block
-// would need a fold over 43 904 of them, 0.057 ms per step on one block.
-template <typename R>
-__global__ void __launch_bounds__(256) k_thermal_temperature(const ThermalArgs a) {
-#pragma clang fp contract(off)
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i >= a.N) return;
-  const R* __restrict__ g = (const R*)a.gout;
-  const size_t N = a.N;
-  R T = R(0);
-  bool bad = false;
-#pragma unroll
-  for (int q = 0; q < TQ; ++q) {
-    const R v = g[q * N + i];
-    T = T + v;
-    bad = bad || !(v == v) || fabs(v) > R(1000);
-  }
-  ((R*)a.Tout)[i] = T;
-  bad = bad || T < R(-50) || T > R(150) || !(T == T);
-  const uint64_t cells = __ballot(bad);
-  // the lowest failing lane adds the wave's count
-  if (bad && (cells & ((1ull << (threadIdx.x & 63)) - 1ull)) == 0ull) atomicAdd(a.bad, (uint32_t)__popcll(cells));
-}
-
-// {min, max, sum} of T and, with a velocity, the number of cells with |u| > 1:
-// up to STAT_BLOCKS blocks stride over the field, four values a lane and load
-// where the field's size allows it, and keep their lanes' results in
-// registers, so the field is read at memory speed and 1024 rows are left to
-// fold.  (One value a lane with a row per 256 cells was bound by its FP64
-// shuffles: 0.074 ms for 45 MB, and 0.057 ms to fold 43 904 rows.)
-constexpr uint32_t STAT_BLOCKS = 1024;
-constexpr int STAT_ROW = 4;
-
-template <typename R>
-__device__ inline void load_quad(const R* __restrict__ p, uint32_t j, R (&v)[4]) {
-  if constexpr (sizeof(R) == 4) {
-    const float4 t = ((const float4*)p)[j];
-    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-  } else {
-    const double2 t0 = ((const double2*)p)[2 * (size_t)j], t1 = ((const double2*)p)[2 * (size_t)j + 1];
-    v[0] = t0.x; v[1] = t0.y; v[2] = t1.x; v[3] = t1.y;
-  }
-}
-
-template <typename R, int W>
-__global__ void __launch_bounds__(256) k_thermal_stats(const R* __restrict__ T, const R* __restrict__ u, uint32_t N,
-                                                       double* __restrict__ partial) {
-#pragma clang fp contract(off)
-  double mn = 1.0e300, mx = -1.0e300, sm = 0.0;
-  uint32_t fast = 0;
-  const uint32_t items = N / W;
-  auto one = [&](R t) {
-    const double d = (double)t;
-    mn = fmin(mn, d);
-    mx = fmax(mx, d);
-    sm += d;
-  };
-  auto speed = [&](R x, R y, R z) { fast += sqrt((x * x + y * y) + z * z) > R(1) ? 1u : 0u; };
-  for (uint32_t j = blockIdx.x * 256u + threadIdx.x; j < items; j += gridDim.x * 256u) {
-    if constexpr (W == 4) {
-      R t[4];
-      load_quad<R>(T, j, t);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) one(t[k]);
-      if (u) {
-        R x[4], y[4], z[4];
-        load_quad<R>(u, j, x);
-        load_quad<R>(u + N, j, y);
-        load_quad<R>(u + 2 * (size_t)N, j, z);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) speed(x[k], y[k], z[k]);
-      }
-    } else {
-      one(T[j]);
-      if (u) speed(u[j], u[(size_t)N + j], u[2 * (size_t)N + j]);
-    }
-  }
-  double c = (double)fast;
+// {min, max, sum, count} of the block's lanes into its row of partial.
+__device__ inline void stat_row(double mn, double mx, double sm, double c, double* __restrict__ partial) {
   mn = wave_min(mn);
   mx = wave_max(mx);
   sm = wave_sum(sm);
@@ -248,11 +186,126 @@ __global__ void __launch_bounds__(256) k_thermal_stats(const R* __restrict__ T, 
   }
 }
 
+template <typename R>
+__device__ inline void load_quad(const R* __restrict__ p, uint32_t j, R (&v)[4]) {
+  if constexpr (sizeof(R) == 4) {
+    const float4 t = ((const float4*)p)[j];
+    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+  } else {
+    const double2 t0 = ((const double2*)p)[2 * (size_t)j], t1 = ((const double2*)p)[2 * (size_t)j + 1];
+    v[0] = t0.x; v[1] = t0.y; v[2] = t1.x; v[3] = t1.y;
+  }
+}
+template <typename R>
+__device__ inline void store_quad(R* __restrict__ p, uint32_t j, const R (&v)[4]) {
+  if constexpr (sizeof(R) == 4) {
+    ((float4*)p)[j] = make_float4(v[0], v[1], v[2], v[3]);
+  } else {
+    ((double2*)p)[2 * (size_t)j] = make_double2(v[0], v[1]);
+    ((double2*)p)[2 * (size_t)j + 1] = make_double2(v[2], v[3]);
+  }
+}
+
+// T' = sum_q g'_q and the stability test, W cells a lane and load.  Bound by
+// reading the populations (360 MB at 224^3).  Failing cells are counted in
+// *a.bad, which the collide pass before has set to zero: a wave without one
+// (every wave of a stable state) neither reduces nor stores anything.
+// REP: also the block's {min, max, sum} of T', while they are in registers
+// (a statistics pass over T and u after the step took 0.033 ms at 224^3).
+template <typename R, int W, bool REP>
+__global__ void __launch_bounds__(256) k_thermal_temperature(const ThermalArgs a, double* __restrict__ partial) {
+#pragma clang fp contract(off)
+  const R* __restrict__ gp = (const R*)a.gout;
+  R* __restrict__ Tout = (R*)a.Tout;
+  const size_t N = a.N;
+  const uint32_t items = a.N / W;
+  double mn = 1.0e300, mx = -1.0e300, sm = 0.0;
+  uint32_t nbad = 0;
+  for (uint32_t j = blockIdx.x * 256u + threadIdx.x; j < items; j += gridDim.x * 256u) {
+    R g[TQ][W], T[W];
+#pragma unroll
+    for (int q = 0; q < TQ; ++q) {
+      if constexpr (W == 4) load_quad<R>(gp + q * N, j, g[q]);
+      else g[q][0] = gp[q * N + j];
+    }
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      T[k] = R(0);
+      bool bad = false;
+#pragma unroll
+      for (int q = 0; q < TQ; ++q) {
+        const R v = g[q][k];
+        T[k] = T[k] + v;
+        bad = bad || !(v == v) || fabs(v) > R(1000);
+      }
+      bad = bad || T[k] < R(-50) || T[k] > R(150) || !(T[k] == T[k]);
+      nbad += bad ? 1u : 0u;
+      if constexpr (REP) {
+        const double d = (double)T[k];
+        mn = fmin(mn, d);
+        mx = fmax(mx, d);
+        sm += d;
+      }
+    }
+    if constexpr (W == 4) store_quad<R>(Tout, j, T);
+    else Tout[j] = T[0];
+  }
+  if (__ballot(nbad != 0u) != 0ull) {
+    const double n = wave_sum((double)nbad);
+    if ((threadIdx.x & 63) == 0) atomicAdd(a.bad, (uint32_t)n);
+  }
+  if constexpr (REP) stat_row(mn, mx, sm, 0.0, partial);
+}
+
+// {min, max, sum} of T and, with a velocity, the number of cells with |u| > 1:
+// up to STAT_BLOCKS blocks stride over the field, four values a lane and load
+// where the field's size allows it, and keep their lanes' results in
+// registers, so the field is read at memory speed and 1024 rows are left to
+// fold.  (One value a lane with a row per 256 cells was bound by its FP64
+// shuffles: 0.074 ms for 45 MB, and 0.057 ms to fold 43 904 rows.)
+template <typename R, int W>
+__global__ void __launch_bounds__(256) k_thermal_stats(const R* __restrict__ T, const R* __restrict__ u, uint32_t N,
+                                                       double* __restrict__ partial) {
+#pragma clang fp contract(off)
+  double mn = 1.0e300, mx = -1.0e300, sm = 0.0;
+  uint32_t fast = 0;
+  const uint32_t items = N / W;
+  auto one = [&](R t) {
+    const double d = (double)t;
+    mn = fmin(mn, d);
+    mx = fmax(mx, d);
+    sm += d;
+  };
+  auto speed = [&](R x, R y, R z) { fast += faster_than_one(x, y, z) ? 1u : 0u; };
+  for (uint32_t j = blockIdx.x * 256u + threadIdx.x; j < items; j += gridDim.x * 256u) {
+    if constexpr (W == 4) {
+      R t[4];
+      load_quad<R>(T, j, t);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) one(t[k]);
+      if (u) {
+        R x[4], y[4], z[4];
+        load_quad<R>(u, j, x);
+        load_quad<R>(u + N, j, y);
+        load_quad<R>(u + 2 * (size_t)N, j, z);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) speed(x[k], y[k], z[k]);
+      }
+    } else {
+      one(T[j]);
+      if (u) speed(u[j], u[(size_t)N + j], u[2 * (size_t)N + j]);
+    }
+  }
+  stat_row(mn, mx, sm, (double)fast, partial);
+}
+
 // Fold of at most STAT_BLOCKS rows {min, max, sum, count} into out (pinned host
 // memory): four rows of loads in flight per lane, then across the lanes that
-// hold the same column.
+// hold the same column.  count: {unstable, fast} cells of a reporting step;
+// the fast ones become the fourth value, are cleared for the next step, and
+// the unstable ones follow in out[4].
 __global__ void __launch_bounds__(256) k_thermal_fold(const double* __restrict__ partial, uint32_t rows,
-                                                      double* __restrict__ out) {
+                                                      double* __restrict__ out, uint32_t* __restrict__ count) {
   __shared__ double sh[4][STAT_ROW];
   const int s = threadIdx.x & 3, j = threadIdx.x >> 2;
   auto add = [&](double r, double p) { return s == 0 ? fmin(r, p) : (s == 1 ? fmax(r, p) : r + p); };
@@ -277,7 +330,16 @@ __global__ void __launch_bounds__(256) k_thermal_fold(const double* __restrict__
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if (lane < STAT_ROW) sh[wid][lane] = v;
   __syncthreads();
-  if (threadIdx.x < STAT_ROW) out[threadIdx.x] = add(add(sh[0][s], sh[1][s]), add(sh[2][s], sh[3][s]));
+  if (threadIdx.x < STAT_ROW) {
+    double r = add(add(sh[0][s], sh[1][s]), add(sh[2][s], sh[3][s]));
+    if (count && s == 3) {
+      // one exchange: a plain load here is a scalar one, which the store of
+      // the zero does not wait for
+      r = (double)atomicExch(count + 1, 0u);
+      out[4] = (double)count[0];
+    }
+    out[s] = r;
+  }
 }
 
 template <typename R>
@@ -346,9 +408,21 @@ static void thermal_collide(const ThermalArgs& a, bool first, bool last, dim3 gr
     hipLaunchKernelGGL((k_thermal_collide<R, false, true, false, NT>), grid, dim3(256), 0, s, a);
 }
 
+// Blocks of a pass that strides over the field, W cells a lane.
+static uint32_t stride_blocks(uint32_t N, uint32_t W) { return std::min((N / W + 255u) / 256u, STAT_BLOCKS); }
+
+static bool quad_aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+template <typename R, int W>
+static void thermal_temperature_report(const ThermalArgs& a, double* partial, double* out, hipStream_t s) {
+  const uint32_t blocks = stride_blocks(a.N, W);
+  hipLaunchKernelGGL((k_thermal_temperature<R, W, true>), dim3(blocks), dim3(256), 0, s, a, partial);
+  hipLaunchKernelGGL(k_thermal_fold, dim3(1), dim3(256), 0, s, partial, blocks, out, a.bad);
+}
+
 template <typename R>
 static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void* const T[2], int& gcur, int& tcur,
-                                int nsteps, hipStream_t s) {
+                                int nsteps, double* partial, double* out, hipStream_t s) {
   // With convection a step's source needs the whole temperature field of its
   // input state before it starts, so every step runs the temperature pass.
   // Pure diffusion reads only the cell's own populations: the temperature
@@ -358,7 +432,8 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
   // would be overwritten unread, 4 of 64 B per cell).  A run's first step
   // leaves the input state's temperature as the caller set it (it may be a
   // boundary value rather than sum g).
-  const dim3 grid((base.N + 255) / 256);
+  // four cells a lane when every population plane starts on a 16-byte boundary
+  const bool quad = base.N % 4 == 0 && quad_aligned(g[0]) && quad_aligned(g[1]) && quad_aligned(T[0]) && quad_aligned(T[1]);
   // convection reads the temperature's neighbours (populations, T, u and the
   // sources, 80 B a cell); pure diffusion reads only the cell's own values
   const BlockOrder ord =
@@ -375,7 +450,12 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
     const bool last = n + 1 == nsteps;
     if (nt) thermal_collide<R, true>(a, n == 0, last, cgrid, s);
     else thermal_collide<R, false>(a, n == 0, last, cgrid, s);
-    if (a.conv || last) hipLaunchKernelGGL(k_thermal_temperature<R>, grid, dim3(256), 0, s, a);
+    if (last && a.report) {
+      if (quad) thermal_temperature_report<R, 4>(a, partial, out, s);
+      else thermal_temperature_report<R, 1>(a, partial, out, s);
+    } else if (a.conv || last) {
+      hipLaunchKernelGGL((k_thermal_temperature<R, 1, false>), dim3((a.N + 255) / 256), dim3(256), 0, s, a, nullptr);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     gcur = 1 - gcur;
@@ -385,25 +465,24 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
 }
 
 hipError_t launch_thermal_steps(bool dbl, const ThermalArgs& base, void* const g[2], void* const T[2], int& gcur,
-                                int& tcur, int nsteps, hipStream_t s) {
-  return dbl ? thermal_steps<double>(base, g, T, gcur, tcur, nsteps, s)
-             : thermal_steps<float>(base, g, T, gcur, tcur, nsteps, s);
+                                int& tcur, int nsteps, double* partial, double* out, hipStream_t s) {
+  return dbl ? thermal_steps<double>(base, g, T, gcur, tcur, nsteps, partial, out, s)
+             : thermal_steps<float>(base, g, T, gcur, tcur, nsteps, partial, out, s);
 }
 
 template <typename R>
 static hipError_t thermal_stats(const void* T, const void* u, uint32_t N, double* partial, double* out, hipStream_t s) {
   // four values a load when every component of u starts on a 16-byte
   // boundary (N % 4; the bases are allocations or whole multiples of it)
-  const bool quad = N % 4 == 0 && ((uintptr_t)T & 15) == 0 && ((uintptr_t)u & 15) == 0;
-  const uint32_t items = quad ? N / 4 : N;
-  const uint32_t blocks = std::min((items + 255u) / 256u, STAT_BLOCKS);
+  const bool quad = N % 4 == 0 && quad_aligned(T) && quad_aligned(u);
+  const uint32_t blocks = stride_blocks(N, quad ? 4 : 1);
   if (quad)
     hipLaunchKernelGGL((k_thermal_stats<R, 4>), dim3(blocks), dim3(256), 0, s, (const R*)T, (const R*)u, N, partial);
   else
     hipLaunchKernelGGL((k_thermal_stats<R, 1>), dim3(blocks), dim3(256), 0, s, (const R*)T, (const R*)u, N, partial);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_thermal_fold, dim3(1), dim3(256), 0, s, partial, blocks, out);
+  hipLaunchKernelGGL(k_thermal_fold, dim3(1), dim3(256), 0, s, partial, blocks, out, (uint32_t*)nullptr);
   return hipGetLastError();
 }
 

@@ -196,19 +196,28 @@ class ThermalLBM:
         """thermal_lbm.py:396-427: True when the stability test passes."""
         return self._step(None)
 
-    def step_with_velocity(self, velocity_field) -> bool:
+    def step_with_velocity(self, velocity_field, stats: Optional[np.ndarray] = None) -> bool:
         """set_velocity_field(velocity_field) and step() in one: with
         convection on, a device velocity of the solver's type and layout is
-        copied inside the step."""
+        copied inside the step.  stats (float64 [4]): the step's coupling
+        statistics, formed inside it where the velocity is."""
         src = self._velocity_source(velocity_field)
         v = self._vel
         if (self.is_initialized and self.enable_convection and isinstance(src, torch.Tensor) and src.device == v.device
                 and src.dtype == v.dtype and src.shape == v.shape and src.is_contiguous()):
-            return self._step(src)
+            return self._step(src, stats)
         self.set_velocity_field(src)
-        return self._step(None)
+        ok = self._step(None)
+        if ok and stats is not None:
+            self._coupling_stats(stats)
+        return ok
 
-    def _step(self, velocity: Optional[torch.Tensor]) -> bool:
+    def _coupling_stats(self, out: np.ndarray) -> None:
+        """{min, max, sum} of T and the number of cells with |u| > 1 into out (float64 [4])."""
+        L.check(self.lib.pol_thermal_coupling_stats(self.ctx.handle, out.ctypes.data, L.stream_handle()),
+                self.ctx.handle, "pol_thermal_coupling_stats")
+
+    def _step(self, velocity: Optional[torch.Tensor], stats: Optional[np.ndarray] = None) -> bool:
         if not self.is_initialized:
             return False
         u = C.c_int32()
@@ -216,6 +225,7 @@ class ThermalLBM:
             st = self.lib.pol_thermal_step(self.ctx.handle, 1, C.byref(u), L.stream_handle())
         else:
             st = self.lib.pol_thermal_step_with_velocity(self.ctx.handle, 1, velocity.data_ptr(), C.byref(u),
+                                                         None if stats is None else stats.ctypes.data,
                                                          L.stream_handle())
         L.check(st, self.ctx.handle, "pol_thermal_step")
         self._gcur ^= 1
@@ -439,23 +449,30 @@ class ThermalFluidCoupledSolver:
         t2 = time.time()
         if not self.fused_reset:
             self.thermal_solver.reset_heat_source_to_base(self.base_heat_source)
+        figures = None  # of the check below, where a step forms them itself
         for k in range(cfg.thermal_subcycles):
-            hand_over = k == 0 and velocity is not None
-            if not (self.thermal_solver.step_with_velocity(velocity) if hand_over else self.thermal_solver.step()):
+            if k == 0 and velocity is not None:
+                if cfg.enable_diagnostics and cfg.thermal_subcycles == 1:
+                    figures = np.zeros(4, dtype=np.float64)
+                ok = self.thermal_solver.step_with_velocity(velocity, figures)
+            else:
+                ok = self.thermal_solver.step()
+            if not ok:
                 return False
         self.performance_stats["thermal_time"] += time.time() - t2
-        if cfg.enable_diagnostics and not self._check_coupling_stability():
+        if cfg.enable_diagnostics and not self._check_coupling_stability(figures):
             return False
         self.coupling_step += 1
         self.performance_stats["total_steps"] += 1
         return True
 
-    def _check_coupling_stability(self) -> bool:
-        """thermal_fluid_coupled.py:237-262, its figures from one device pass."""
-        th = self.thermal_solver
-        out = np.zeros(4, dtype=np.float64)
-        L.check(th.lib.pol_thermal_coupling_stats(th.ctx.handle, out.ctypes.data, L.stream_handle()), th.ctx.handle,
-                "pol_thermal_coupling_stats")
+    def _check_coupling_stability(self, figures: Optional[np.ndarray] = None) -> bool:
+        """thermal_fluid_coupled.py:237-262, its figures from one device pass
+        or from the step (`figures`)."""
+        out = figures
+        if out is None:
+            out = np.zeros(4, dtype=np.float64)
+            self.thermal_solver._coupling_stats(out)
         tmin, tmax, _, fast_cells = (float(v) for v in out)
         if tmax > 150.0 or tmin < -10.0:
             return False

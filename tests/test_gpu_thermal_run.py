@@ -131,3 +131,34 @@ def test_streaming_steps(precision, shape, convection):
     assert np.array_equal(a.g, st["g"]) and np.array_equal(a.temperature.to_numpy(), st["T"])
     assert np.array_equal(a.temperature_old.to_numpy(), st["T_old"])
     assert np.array_equal(a.heat_source.to_numpy(), st["heat_source"])
+
+
+@pytest.mark.parametrize("precision", ["f32", "f64"])
+@pytest.mark.parametrize("shape", SHAPES + [(128, 64, 33), (101, 103, 107)])
+def test_statistics_of_the_step(shape, precision):
+    """A step's own coupling statistics: those of the pass over its result, and
+    afresh after a step with fast cells (|u| just at, next to and above 1)."""
+    print("case: statistics of the step %s %s" % (shape, precision), flush=True)
+    th = _make(shape, precision, True)
+    n, eps = th._hs.numel(), np.finfo(np.float64).eps
+    rng = np.random.default_rng(17)
+    one = th._hs.new_ones(1)
+    after = torch.nextafter(one, 2 * one)  # a square of it is above one, its root rounds to it
+    for speeds in ([], [one, -one], [after], [3 * one, float("nan") * one, float("inf") * one], []):
+        u = torch.from_numpy(rng.uniform(-0.02, 0.02, tuple(th._vel.shape))).to(th._vel)
+        cells = rng.choice(n, len(speeds), replace=False)
+        for c, v in zip(cells, speeds):
+            u.view(3, -1)[:, c] = 0.0
+            u.view(3, -1)[rng.integers(3), c] = v
+        got, want = np.zeros(4), np.zeros(4)
+        th.initialize_from(rng.uniform(20.0, 90.0, shape))
+        ok = th.step_with_velocity(u, got)
+        th._coupling_stats(want)
+        uu = u.view(3, -1).cpu().numpy()
+        assert want[3] == (np.sqrt((uu[0] * uu[0] + uu[1] * uu[1]) + uu[2] * uu[2]) > 1).sum()
+        T = th.temperature.to_torch().double().cpu().numpy()
+        bad = (th.g_device.isnan() | (th.g_device.abs() > 1000)).any(dim=0).cpu().numpy() | ~((T >= -50) & (T <= 150))
+        assert th._last_unstable == int(bad.sum()) and ok == (not bad.any())
+        assert np.array_equal(got[[0, 1, 3]], want[[0, 1, 3]])
+        if np.isfinite(T).all():
+            assert abs(got[2] - want[2]) <= 2 * n * eps * np.abs(T).sum()  # any order of the sum
