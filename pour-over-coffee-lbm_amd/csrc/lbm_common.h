@@ -242,6 +242,12 @@ inline BlockOrder stencil_order(uint64_t cells, uint64_t bytes) {
 inline uint32_t launch_blocks(const BlockOrder& o) { return launch_blocks(o.order, Grid{o.nblk, o.per_xcd, o.per_xcd * NXCD}); }
 __device__ inline uint32_t ordered_block(const BlockOrder& o) { return ordered_block(o.order, o.per_xcd); }
 
+// A load that leaves the caches to others (NT) or an ordinary one.
+template <bool NT, typename T>
+__device__ inline T load_as(const T* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
 // A store that leaves the caches to others (NT) or an ordinary one.
 template <bool NT, typename T>
 __device__ inline void store_as(T* p, T v) {

@@ -73,11 +73,15 @@ __device__ inline void decompose(const ThermalArgs& a, uint32_t i, uint32_t& x, 
 // HAND: the velocity comes from a.u_src (the fluid's field) and is stored to
 // a.u beside the step, instead of a copy before it (270 MB and 0.085 ms at
 // 224^3; here its read is the one the convection needs anyway, 0.03 ms more).
-// NT (populations above the last-level cache): the heat source, the rest and
-// the y and z populations are stored past the cache (224^3: diffusion step
-// 135.3 -> 132.7 us, 187 x 150 x 201: 66.4 -> 61.1).  The x populations, whose
-// one-cell shift splits a sector at both ends of every wave, stay cached
-// (streamed as well: diffusion 63.2 us, convection collide pass 173 -> 187).
+// NT (populations above the last-level cache): what this pass reads for the
+// last time or writes for a later step bypasses the cache: the populations it
+// reads, the rest and the y and z populations it writes, the sources, the
+// velocity handed over.  The temperature's neighbours and the x populations
+// written stay cached (their one-cell shift splits a sector at both ends of
+// every wave: streamed as well, diffusion at 187 x 150 x 201 63.2 us, convection
+// collide pass at 224^3 173 -> 187).  Stores alone: diffusion 66.4 -> 61.1 us,
+// 224^3 135.3 -> 132.7.  Loads and the velocity too, coupled step at 224^3: this
+// pass 173 -> 160 us, the fluid step after it 116 -> 108.
 template <typename R, bool CONV, bool WT, bool HAND, bool NT>
 __global__ void __launch_bounds__(256) k_thermal_collide(const ThermalArgs a) {
 #pragma clang fp contract(off)
@@ -93,25 +97,25 @@ __global__ void __launch_bounds__(256) k_thermal_collide(const ThermalArgs a) {
   const size_t N = a.N;
   R g[TQ];
 #pragma unroll
-  for (int q = 0; q < TQ; ++q) g[q] = gin[q * N + i];
+  for (int q = 0; q < TQ; ++q) g[q] = load_as<NT>(gin + q * N + i);
   R T = R(0);
 #pragma unroll
   for (int q = 0; q < TQ; ++q) T = T + g[q];
   if constexpr (WT) ((R*)a.T)[i] = T;
   R* __restrict__ hs = (R*)a.hs;
   const R* __restrict__ hsb = (const R*)a.hsb;
-  R S = hsb ? hsb[i] : hs[i];
+  R S = hsb ? load_as<NT>(hsb + i) : hs[i];
   bool write_s = hsb != nullptr;
   R v0 = R(0), v1 = R(0), v2 = R(0);
   if constexpr (HAND) {  // each cell reads and writes its own elements only: u_src may be u
     const R* us = (const R*)a.u_src;
-    v0 = us[i];
-    v1 = us[N + i];
-    v2 = us[2 * N + i];
+    v0 = load_as<NT>(us + i);
+    v1 = load_as<NT>(us + N + i);
+    v2 = load_as<NT>(us + 2 * N + i);
     R* u = (R*)a.u;
-    u[i] = v0;
-    u[N + i] = v1;
-    u[2 * N + i] = v2;
+    store_as<NT>(u + i, v0);
+    store_as<NT>(u + N + i, v1);
+    store_as<NT>(u + 2 * N + i, v2);
     if (a.report) {  // cells with |u| > 1: zero on entry, taken and cleared by the fold
       const bool fast = faster_than_one(v0, v1, v2);
       const uint64_t cells = __ballot(fast);
@@ -187,22 +191,37 @@ __device__ inline void stat_row(double mn, double mx, double sm, double c, doubl
 }
 
 template <typename R>
+struct Vec16;  // 16 bytes
+template <>
+struct Vec16<float> {
+  typedef float type __attribute__((ext_vector_type(4)));
+};
+template <>
+struct Vec16<double> {
+  typedef double type __attribute__((ext_vector_type(2)));
+};
+// Values 4 j .. 4 j + 3 of p (16-byte aligned).
+template <bool NT = false, typename R>
 __device__ inline void load_quad(const R* __restrict__ p, uint32_t j, R (&v)[4]) {
-  if constexpr (sizeof(R) == 4) {
-    const float4 t = ((const float4*)p)[j];
-    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-  } else {
-    const double2 t0 = ((const double2*)p)[2 * (size_t)j], t1 = ((const double2*)p)[2 * (size_t)j + 1];
-    v[0] = t0.x; v[1] = t0.y; v[2] = t1.x; v[3] = t1.y;
+  using V = typename Vec16<R>::type;
+  constexpr int W = 16 / sizeof(R);
+#pragma unroll
+  for (int k = 0; k < 4; k += W) {
+    const V t = load_as<NT>((const V*)(p + 4 * (size_t)j + k));
+#pragma unroll
+    for (int l = 0; l < W; ++l) v[k + l] = t[l];
   }
 }
-template <typename R>
+template <bool NT, typename R>
 __device__ inline void store_quad(R* __restrict__ p, uint32_t j, const R (&v)[4]) {
-  if constexpr (sizeof(R) == 4) {
-    ((float4*)p)[j] = make_float4(v[0], v[1], v[2], v[3]);
-  } else {
-    ((double2*)p)[2 * (size_t)j] = make_double2(v[0], v[1]);
-    ((double2*)p)[2 * (size_t)j + 1] = make_double2(v[2], v[3]);
+  using V = typename Vec16<R>::type;
+  constexpr int W = 16 / sizeof(R);
+#pragma unroll
+  for (int k = 0; k < 4; k += W) {
+    V t;
+#pragma unroll
+    for (int l = 0; l < W; ++l) t[l] = v[k + l];
+    store_as<NT>((V*)(p + 4 * (size_t)j + k), t);
   }
 }
 
@@ -212,7 +231,11 @@ __device__ inline void store_quad(R* __restrict__ p, uint32_t j, const R (&v)[4]
 // (every wave of a stable state) neither reduces nor stores anything.
 // REP: also the block's {min, max, sum} of T', while they are in registers
 // (a statistics pass over T and u after the step took 0.033 ms at 224^3).
-template <typename R, int W, bool REP>
+// NT (populations above the last-level cache): nothing here is read again
+// before the cache has turned over, so loads and stores bypass it (reporting
+// pass at 224^3 85 -> 67 us; cached, its loads also evict what the fluid step
+// that follows would find).
+template <typename R, int W, bool REP, bool NT>
 __global__ void __launch_bounds__(256) k_thermal_temperature(const ThermalArgs a, double* __restrict__ partial) {
 #pragma clang fp contract(off)
   const R* __restrict__ gp = (const R*)a.gout;
@@ -225,8 +248,8 @@ __global__ void __launch_bounds__(256) k_thermal_temperature(const ThermalArgs a
     R g[TQ][W], T[W];
 #pragma unroll
     for (int q = 0; q < TQ; ++q) {
-      if constexpr (W == 4) load_quad<R>(gp + q * N, j, g[q]);
-      else g[q][0] = gp[q * N + j];
+      if constexpr (W == 4) load_quad<NT>(gp + q * N, j, g[q]);
+      else g[q][0] = load_as<NT>(gp + q * N + j);
     }
 #pragma unroll
     for (int k = 0; k < W; ++k) {
@@ -247,8 +270,8 @@ __global__ void __launch_bounds__(256) k_thermal_temperature(const ThermalArgs a
         sm += d;
       }
     }
-    if constexpr (W == 4) store_quad<R>(Tout, j, T);
-    else Tout[j] = T[0];
+    if constexpr (W == 4) store_quad<NT>(Tout, j, T);
+    else store_as<NT>(Tout + j, T[0]);
   }
   if (__ballot(nbad != 0u) != 0ull) {
     const double n = wave_sum((double)nbad);
@@ -280,14 +303,14 @@ __global__ void __launch_bounds__(256) k_thermal_stats(const R* __restrict__ T, 
   for (uint32_t j = blockIdx.x * 256u + threadIdx.x; j < items; j += gridDim.x * 256u) {
     if constexpr (W == 4) {
       R t[4];
-      load_quad<R>(T, j, t);
+      load_quad(T, j, t);
 #pragma unroll
       for (int k = 0; k < 4; ++k) one(t[k]);
       if (u) {
         R x[4], y[4], z[4];
-        load_quad<R>(u, j, x);
-        load_quad<R>(u + N, j, y);
-        load_quad<R>(u + 2 * (size_t)N, j, z);
+        load_quad(u, j, x);
+        load_quad(u + N, j, y);
+        load_quad(u + 2 * (size_t)N, j, z);
 #pragma unroll
         for (int k = 0; k < 4; ++k) speed(x[k], y[k], z[k]);
       }
@@ -413,10 +436,20 @@ static uint32_t stride_blocks(uint32_t N, uint32_t W) { return std::min((N / W +
 
 static bool quad_aligned(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-template <typename R, int W>
-static void thermal_temperature_report(const ThermalArgs& a, double* partial, double* out, hipStream_t s) {
-  const uint32_t blocks = stride_blocks(a.N, W);
-  hipLaunchKernelGGL((k_thermal_temperature<R, W, true>), dim3(blocks), dim3(256), 0, s, a, partial);
+// The temperature pass: with its statistics (partial not null) striding, four
+// cells a lane where every plane starts on a 16-byte boundary, so that few
+// rows are left to fold; else one cell a lane (striding: 31.3 -> 33.8 us at
+// 187 x 150 x 201).
+template <typename R, bool NT>
+static void thermal_temperature(const ThermalArgs& a, double* partial, double* out, hipStream_t s) {
+  if (!partial) {
+    hipLaunchKernelGGL((k_thermal_temperature<R, 1, false, NT>), dim3((a.N + 255) / 256), dim3(256), 0, s, a, nullptr);
+    return;
+  }
+  const bool quad = a.N % 4 == 0 && quad_aligned(a.gout) && quad_aligned(a.Tout);
+  const uint32_t blocks = stride_blocks(a.N, quad ? 4 : 1);
+  if (quad) hipLaunchKernelGGL((k_thermal_temperature<R, 4, true, NT>), dim3(blocks), dim3(256), 0, s, a, partial);
+  else hipLaunchKernelGGL((k_thermal_temperature<R, 1, true, NT>), dim3(blocks), dim3(256), 0, s, a, partial);
   hipLaunchKernelGGL(k_thermal_fold, dim3(1), dim3(256), 0, s, partial, blocks, out, a.bad);
 }
 
@@ -432,8 +465,6 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
   // would be overwritten unread, 4 of 64 B per cell).  A run's first step
   // leaves the input state's temperature as the caller set it (it may be a
   // boundary value rather than sum g).
-  // four cells a lane when every population plane starts on a 16-byte boundary
-  const bool quad = base.N % 4 == 0 && quad_aligned(g[0]) && quad_aligned(g[1]) && quad_aligned(T[0]) && quad_aligned(T[1]);
   // convection reads the temperature's neighbours (populations, T, u and the
   // sources, 80 B a cell); pure diffusion reads only the cell's own values
   const BlockOrder ord =
@@ -450,11 +481,10 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
     const bool last = n + 1 == nsteps;
     if (nt) thermal_collide<R, true>(a, n == 0, last, cgrid, s);
     else thermal_collide<R, false>(a, n == 0, last, cgrid, s);
-    if (last && a.report) {
-      if (quad) thermal_temperature_report<R, 4>(a, partial, out, s);
-      else thermal_temperature_report<R, 1>(a, partial, out, s);
-    } else if (a.conv || last) {
-      hipLaunchKernelGGL((k_thermal_temperature<R, 1, false>), dim3((a.N + 255) / 256), dim3(256), 0, s, a, nullptr);
+    double* const rows = last && a.report ? partial : nullptr;
+    if (a.conv || last) {
+      if (nt) thermal_temperature<R, true>(a, rows, out, s);
+      else thermal_temperature<R, false>(a, rows, out, s);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

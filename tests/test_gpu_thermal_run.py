@@ -162,3 +162,27 @@ def test_statistics_of_the_step(shape, precision):
         assert np.array_equal(got[[0, 1, 3]], want[[0, 1, 3]])
         if np.isfinite(T).all():
             assert abs(got[2] - want[2]) <= 2 * n * eps * np.abs(T).sum()  # any order of the sum
+
+
+@pytest.mark.parametrize("precision,shape", [("f32", (171, 168, 173)), ("f32", (171, 167, 175)), ("f64", (131, 130, 145)),
+                                             ("f64", (131, 131, 145))])
+def test_streaming_step_with_velocity(precision, shape):
+    """The hand-over and the statistics of a step past the cache, in cell counts
+    that are and are not a multiple of four."""
+    print("case: streaming step with velocity %s %s" % (shape, precision), flush=True)
+    a, b = _make(shape, precision, True), _make(shape, precision, True)
+    assert 2 * a.g_device.numel() * a.g_device.element_size() > 256 << 20
+    u = torch.from_numpy(np.random.default_rng(11).uniform(-0.02, 0.02, tuple(a._vel.shape))).to(a._vel)
+    u.view(3, -1)[0, -3:] = 1.5
+    for th in (a, b):
+        th.use_base_heat_source(torch.full_like(th._hs, 1e-3))
+    got, want = np.zeros(4), np.zeros(4)
+    ok = a.step_with_velocity(u, got)
+    b.set_velocity_field(u)
+    assert ok and b.step()
+    for x, y in ((a._vel, b._vel), (a.g_device, b.g_device), (a._hs, b._hs), (a._T[a._tcur], b._T[b._tcur])):
+        assert torch.equal(x, y)
+    b._coupling_stats(want)
+    assert np.array_equal(got[[0, 1, 3]], want[[0, 1, 3]]) and got[3] == 3
+    n, eps = b._hs.numel(), np.finfo(np.float64).eps
+    assert abs(got[2] - want[2]) <= 2 * n * eps * abs(want[2])  # positive terms, any order
