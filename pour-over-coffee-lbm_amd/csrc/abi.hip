@@ -316,6 +316,21 @@ static StepArgs make_args(const pol_ctx* c, const void* fin, void* fout, uint32_
   const bool streams = 2ull * a.n_items * Q * storage_bytes(d.storage) > (256ull << 20);
   const bool whole_sectors = a.chunks || ((uint64_t)c->P * storage_bytes(d.storage)) % 64 == 0;
   a.stream_store = streams && whole_sectors ? 1u : 0u;
+  // A streaming step of the compact layout that applies the particle drag field
+  // also pulls its populations past the cache where they and the eight fields
+  // of the coupling (drag, rho, u) do not fit it together but the fields alone
+  // do: those are what the next coupling pass and step read again.  Coupled
+  // step FP32 at 200^3 / 224^3 / 256^3 120 -> 116 / 188 -> 169 / 262 -> 250 us
+  // (280^3 no change), FP64 at 160^3 / 224^3 130 -> 122 / 328 -> 311.  Outside of
+  // that it costs: FP32 192^3 (all fits) 114 -> 117, 320^3 (the fields do not)
+  // 462 -> 500, FP16 288^3 (issue bound)
+  // 239 -> 245; without the drag field 106 -> 115 at 224^3 FP32.
+  const size_t rb = storage_bytes(d.storage) == 8 ? 8 : 4;
+  const uint64_t pulled = (uint64_t)a.n_items * Q * storage_bytes(d.storage), fields = (uint64_t)a.n_items * 8 * rb;
+  a.stream_pull = a.stream_store && a.records && (d.options & POL_PARTICLE_FIELD) && storage_bytes(d.storage) >= 4 &&
+                          pulled + fields > LAST_LEVEL_BYTES && fields <= LAST_LEVEL_BYTES
+                      ? 1u
+                      : 0u;
   // Streaming steps sweep one memory front: linear blocks over the dense
   // grid, groups of 4 consecutive blocks per XCD over the compact chunk list,
   // groups of 32 where split sectors have to meet in an L2 (the sizes above,

@@ -55,7 +55,9 @@ struct CompactRows {
 // flags is set.
 // RAW: hand use() the stored value itself instead of its decoded real.
 // SKIP: test per wave whether any lane has a bounce link (see below).
-template <typename S, bool A32, bool XF, bool RAW = false, bool SKIP = (sizeof(S) == 2), typename Use>
+// PULL_NT: loads that leave the last-level cache to others.
+template <typename S, bool A32, bool XF, bool RAW = false, bool SKIP = (sizeof(S) == 2), bool PULL_NT = false,
+          typename Use>
 __device__ __forceinline__ void compact_sources(const S* __restrict__ fin, uint32_t PS, const int (&rb)[9], uint32_t x,
                                                 uint32_t nx, bool px, uint32_t own, uint32_t fl, Use&& use) {
   using C = Codec<S>;
@@ -91,7 +93,7 @@ __device__ __forceinline__ void compact_sources(const S* __restrict__ fin, uint3
         off = (bounce & m) | (off & ~m);
       }
       const S* base = fin + (AI)lo * PS;
-      const S v = *((const S*)((const char*)base + off) + (1 - EX(q)));
+      const S v = load_as<PULL_NT>((const S*)((const char*)base + off) + (1 - EX(q)));
       if constexpr (RAW) use(qc, v);
       else use(qc, C::decode(v));
     });

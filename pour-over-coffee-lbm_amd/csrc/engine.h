@@ -35,6 +35,7 @@ struct StepArgs {
   uint32_t n_items;        // number of work items (cells, or chunk cells x chunks)
   uint32_t cshift;         // log2 of the cells per chunk
   uint32_t stream_store;   // select the non-temporal-store kernels (output far above the last-level cache)
+  uint32_t stream_pull;    // also pull the populations past the last-level cache (compact layout, 4- and 8-byte storage)
   uint32_t xface;          // compact layout: some run reaches x = 0 or nx - 1 (gather wraps / clamps x there)
   uint32_t N, nx, ny, nz, nxy;
   FastDiv dnx, dny;

@@ -20,7 +20,10 @@ namespace pol {
 template <typename S, bool A32, bool XF>
 static void launch_sparse(const StepArgs& a, bool store_f, dim3 grid, hipStream_t s) {
   dim3 block(BLOCK);
-  if (store_f && a.stream_store) {
+  if (store_f && a.stream_store && a.stream_pull) {
+    if constexpr (sizeof(S) >= 4)  // the only storages that stream_pull is set for
+      hipLaunchKernelGGL((k_stream_collide<S, true, true, true, A32, true, true, XF, true, true>), grid, block, 0, s, a);
+  } else if (store_f && a.stream_store) {
     hipLaunchKernelGGL((k_stream_collide<S, true, true, true, A32, true, true, XF>), grid, block, 0, s, a);
   } else if (store_f) {
     hipLaunchKernelGGL((k_stream_collide<S, true, true, true, A32, false, true, XF>), grid, block, 0, s, a);

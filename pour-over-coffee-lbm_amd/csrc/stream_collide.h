@@ -51,8 +51,9 @@ __device__ inline Phys<R> make_phys(const StepArgs& a) {
 // COLLIDE = false: collisionless streaming (f_out = the gathered populations,
 // bounce-back links and open faces as in a step), the step's memory access
 // pattern with none of its arithmetic.
+// PULL_NT: the compact gather bypasses the last-level cache (a.stream_pull).
 template <typename S, bool FLAGS, bool FULL, bool STORE, bool A32, bool NT = false, bool SPARSE = false, bool XF = true,
-          bool COLLIDE = true>
+          bool COLLIDE = true, bool PULL_NT = false>
 __global__ void __launch_bounds__(BLOCK) k_stream_collide(const StepArgs a) {
   static_assert(!SPARSE || (FLAGS && FULL), "the compact layout runs the general kernel");
   using C = Codec<S>;
@@ -111,7 +112,7 @@ __global__ void __launch_bounds__(BLOCK) k_stream_collide(const StepArgs a) {
                                             });
           f[0] = (R)__builtin_bit_cast(_Float16, (uint16_t)h[0]);
         } else {
-          compact_sources<S, A32, XF, false, COLLIDE && sizeof(S) == 2>(
+          compact_sources<S, A32, XF, false, COLLIDE && sizeof(S) == 2, PULL_NT>(
               fin, PS, rb, x, a.nx, (a.options & POL_PERIODIC_X) != 0, own, fl,
               [&](auto qc, R v) { f[decltype(qc)::value] = v; });
         }
