@@ -133,9 +133,10 @@ __global__ void __launch_bounds__(256) k_mp_interface(const MultiphaseArgs a) {
 
 // NT (fields above the last-level cache): the three outputs are read a whole
 // main-loop step later and are stored past the cache, which then still holds
-// the force, u and rho that the passes between them share.  The pass itself
-// gains nothing (75 us at 224^3 either way), the main-loop step 9 us of its
-// 130 us fluid step and 2 us of the velocity pass.
+// the force, u and rho that the passes between them share, and u is read here
+// for the last time before the fluid step rewrites it.  The stores alone: the
+// pass itself 75 us at 224^3 either way, the fluid step 130 -> 121 us and the
+// velocity pass 88 -> 86; the loads: pass 76.1 -> 74.6, fluid step 120.8 -> 119.0.
 template <typename R, bool NT>
 __global__ void __launch_bounds__(256) k_mp_phase(const MultiphaseArgs a) {
 #pragma clang fp contract(off)
@@ -154,7 +155,9 @@ __global__ void __launch_bounds__(256) k_mp_phase(const MultiphaseArgs a) {
     const float pxm = phi[i - 1], pxp = phi[i + 1];
     const float pym = phi[i - a.nx], pyp = phi[i + a.nx];
     const float pzm = phi[i - a.nxy], pzp = phi[i + a.nxy];
-    const float ux = ld_real<R>(a.u, i), uy = ld_real<R>(a.u, N + i), uz = ld_real<R>(a.u, 2 * N + i);
+    const R* u = (const R*)a.u;
+    const float ux = (float)load_as<NT>(u + i), uy = (float)load_as<NT>(u + N + i),
+                uz = (float)load_as<NT>(u + 2 * N + i);
     const float dx = ux > 0.0f ? p - pxm : pxp - p;
     const float dy = uy > 0.0f ? p - pym : pyp - p;
     const float dz = uz > 0.0f ? p - pzm : pzp - p;
