@@ -414,11 +414,11 @@ def bench_diagnostics(reps=200, host=True):
 # reads g (7 x 4) and writes T (4).  Convection adds T (4, the stencil counted
 # once), u (3 x 4) and the heat-source write (4) to the collide pass (the
 # base heat source is read in place of the heat source) and runs the
-# temperature pass every step: 112 B.  Pure diffusion stores T in the next
-# collide pass (+4 B) and runs the temperature pass once per run: 64 B per
-# step + 32 B per run.
+# temperature pass every step: 112 B.  Pure diffusion stores T in the
+# last collide pass of a run (+4 B) and runs the temperature pass once per run:
+# 60 B per step + 36 B per run.
 def thermal_bytes(conv: bool, steps: int) -> float:
-    return 112.0 if conv else 64.0 + 32.0 / steps
+    return 112.0 if conv else 60.0 + 36.0 / steps
 
 
 def bench_thermal(n=224, steps=200, warmup=20, cpu=True):

@@ -13,7 +13,9 @@
  * asynchronously on the hipStream_t passed as `stream` (NULL = legacy
  * default stream); only entry points that hand results back to host memory
  * (pol_reduce, pol_macroscopic / pol_step_ex / pol_step_from with a
- * reduction, pol_adjoint_collect) synchronise that stream.
+ * reduction, pol_step_record with objective steps, pol_adjoint_collect,
+ * pol_field_stats, the thermal statistics, thermal steps with a stability
+ * count or statistics) synchronise that stream.
  *
  * The reference (latteine1217/pour-over-coffee-lbm) is Python + Taichi and
  * has no C ABI; each entry point below names the reference interface whose
