@@ -40,7 +40,7 @@ struct pol_ctx {
   uint32_t stat_tiles = 0;          // blocks per z plane
   double* stat_partial = nullptr;   // [nz * stat_tiles][POL_NSTAT]
   double* stat_zpart = nullptr;     // [nz * stat_tiles]
-  double* stat_dev = nullptr;       // [POL_NSTAT + nz]
+  unsigned long long* pop_dev = nullptr;  // [2] NaN, Inf populations of the scan (zero between calls)
   // multiphase phase field
   bool mp = false;
   pol_multiphase_desc md{};
@@ -149,7 +149,9 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
   const size_t sblk = (size_t)c->stat_tiles * d.nz;
   if (e == hipSuccess) e = hipMalloc((void**)&c->stat_partial, sblk * POL_NSTAT * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&c->stat_zpart, sblk * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void**)&c->stat_dev, ((size_t)POL_NSTAT + d.nz) * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc((void**)&c->pop_dev, 2 * sizeof(unsigned long long));
+  const unsigned long long nopop[2] = {0ull, 0ull};
+  if (e == hipSuccess) e = hipMemcpy(c->pop_dev, nopop, sizeof(nopop), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipHostMalloc((void**)&c->host, ((size_t)POL_NSTAT + d.nz) * sizeof(double));
   if (e != hipSuccess) {
     (void)hipHostFree(c->host);
@@ -158,7 +160,7 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
     (void)hipFree(c->adj_partial);
     (void)hipFree(c->stat_partial);
     (void)hipFree(c->stat_zpart);
-    (void)hipFree(c->stat_dev);
+    (void)hipFree(c->pop_dev);
     delete c;
     return POL_ERR_ALLOC;
   }
@@ -174,7 +176,7 @@ int pol_destroy(pol_ctx* c) {
   (void)hipFree(c->adj_partial);
   (void)hipFree(c->stat_partial);
   (void)hipFree(c->stat_zpart);
-  (void)hipFree(c->stat_dev);
+  (void)hipFree(c->pop_dev);
   (void)hipHostFree(c->host);
   delete c;
   return POL_OK;
@@ -908,14 +910,12 @@ int pol_field_stats(pol_ctx* c, const pol_stats_opts* o, double* out, double* z_
   s.partial = c->stat_partial;
   s.zpart = c->stat_zpart;
   hipError_t e = hipSetDevice(d.device);
-  if (e == hipSuccess) e = launch_field_stats(d.storage == POL_F64, s, c->stat_dev, c->stat_dev + POL_NSTAT, st);
+  if (e == hipSuccess) e = launch_field_stats(d.storage == POL_F64, s, st);
   if (e == hipSuccess && o->with_populations) {
     const StepArgs a = make_args(c, c->b.f[c->cur], nullptr, 0u);
-    e = launch_pop_nonfinite(d.storage, a, c->stat_dev, c->wgrid, st);
+    e = launch_pop_nonfinite(d.storage, a, c->pop_dev, c->wgrid, st);
   }
-  // one transfer of statistics and profile into pinned memory, then host copies
-  const size_t nstat = (size_t)POL_NSTAT + (z_profile ? d.nz : 0);
-  if (e == hipSuccess) e = hipMemcpyAsync(c->host, c->stat_dev, nstat * sizeof(double), hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) e = launch_stats_final(s, z_profile != nullptr, c->host, o->with_populations ? c->pop_dev : nullptr, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) return hip_fail(c, e, "pol_field_stats");
   std::memcpy(out, c->host, POL_NSTAT * sizeof(double));

@@ -482,10 +482,14 @@ __global__ void __launch_bounds__(BLOCK, (sizeof(R) == 4 && !EXTRA) ? 8 : 1) k_f
 // Fold the block partials: block s < POL_NSTAT folds statistic s, block
 // POL_NSTAT + z the tiles of plane z.  Thread t combines the partials
 // t, t + 256, ... in order, then the block combines its threads in a fixed
-// tree: the result does not depend on timing (deterministic).
+// tree: the result does not depend on timing (deterministic).  out and zout are
+// pinned host memory (a copy of them after the fold took 8 us of a call).  pop:
+// the counts of k_pop_nonfinite, taken and cleared for the next scan by one
+// exchange each, or null.
 __global__ void __launch_bounds__(256) k_stats_final(const double* __restrict__ partial,
                                                      const double* __restrict__ zpart, uint32_t nblk, uint32_t tiles,
-                                                     double* __restrict__ out, double* __restrict__ zout) {
+                                                     double* __restrict__ out, double* __restrict__ zout,
+                                                     unsigned long long* __restrict__ pop) {
   const uint32_t b = blockIdx.x;
   const bool stat = b < POL_NSTAT;
   const int s = stat ? (int)b : 0;
@@ -504,6 +508,8 @@ __global__ void __launch_bounds__(256) k_stats_final(const double* __restrict__ 
   if (threadIdx.x == 0) {
     double t = sh[0];
     for (int w = 1; w < 4; ++w) t = stat ? stat_combine(s, t, sh[w]) : t + sh[w];
+    if (pop && stat && (s == POL_STAT_FLUID_POP_NAN || s == POL_STAT_FLUID_POP_INF))
+      t = (double)atomicExch(pop + (s == POL_STAT_FLUID_POP_INF), 0ull);
     if (stat) out[s] = t;
     else zout[b - POL_NSTAT] = t;
   }
@@ -530,8 +536,8 @@ __device__ inline bool work_cell(const StepArgs& a, uint32_t lblk, uint32_t& cel
 }
 
 // NaN / Inf populations of the current state over non-solid cells
-// (numerical_stability.py:92-98), added to out[POL_STAT_FLUID_POP_NAN / _INF]
-// (which k_stats_final has set to zero before, on the same stream).  Bound by
+// (numerical_stability.py:92-98), added to out[2] (zero before; k_stats_final
+// takes them after it, on the same stream).  Bound by
 // reading the populations once (224^3 cup, FP32: 0.051 ms for 285 MB).  A
 // state is finite nearly always, so a wave with nothing to report ends
 // without a reduction, a barrier or a store; one that has something adds its
@@ -539,7 +545,7 @@ __device__ inline bool work_cell(const StepArgs& a, uint32_t lblk, uint32_t& cel
 // partial per block instead needs a fold over all of them: 14 784 pairs at
 // 224^3 took one wave 1.28 ms.
 template <typename S, bool SPARSE>
-__global__ void __launch_bounds__(BLOCK) k_pop_nonfinite(const StepArgs a, double* __restrict__ out) {
+__global__ void __launch_bounds__(BLOCK) k_pop_nonfinite(const StepArgs a, unsigned long long* __restrict__ out) {
   const uint32_t lblk = logical_block(a.per_xcd);
   if (lblk >= a.nblk) return;
   uint32_t cell, own, fl;
@@ -555,8 +561,8 @@ __global__ void __launch_bounds__(BLOCK) k_pop_nonfinite(const StepArgs a, doubl
   if (__ballot(bad != 0u) == 0ull) return;
   bad = wave_reduce(bad, [](uint32_t a, uint32_t b) { return a + b; });
   if ((threadIdx.x & 63) == 0) {
-    if (bad & 0xffffu) unsafeAtomicAdd(out + POL_STAT_FLUID_POP_NAN, (double)(bad & 0xffffu));
-    if (bad >> 16) unsafeAtomicAdd(out + POL_STAT_FLUID_POP_INF, (double)(bad >> 16));
+    if (bad & 0xffffu) atomicAdd(out, (unsigned long long)(bad & 0xffffu));
+    if (bad >> 16) atomicAdd(out + 1, (unsigned long long)(bad >> 16));
   }
 }
 
@@ -625,8 +631,7 @@ static void launch_stats(bool extra, dim3 grid, const StatsArgs& s, hipStream_t 
   else hipLaunchKernelGGL((k_field_stats<R, VEC, false>), grid, dim3(BLOCK), 0, st, s);
 }
 
-hipError_t launch_field_stats(bool real_double, const StatsArgs& s, double* out_dev, double* zout_dev,
-                              hipStream_t st) {
+hipError_t launch_field_stats(bool real_double, const StatsArgs& s, hipStream_t st) {
   const dim3 grid(s.tiles, s.nz);
   // 16-byte loads need every plane (and so every u component) to start on a
   // 4-cell boundary; nx >= 4 keeps a 4-cell group within two rows
@@ -640,22 +645,25 @@ hipError_t launch_field_stats(bool real_double, const StatsArgs& s, double* out_
     if (vec) launch_stats<float, true>(extra, grid, s, st);
     else launch_stats<float, false>(extra, grid, s, st);
   }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_stats_final, dim3(POL_NSTAT + s.nz), dim3(256), 0, st, s.partial, s.zpart, s.tiles * s.nz,
-                     s.tiles, out_dev, zout_dev);
+  return hipGetLastError();
+}
+
+hipError_t launch_stats_final(const StatsArgs& s, bool profile, double* out, unsigned long long* pop, hipStream_t st) {
+  hipLaunchKernelGGL(k_stats_final, dim3(POL_NSTAT + (profile ? s.nz : 0)), dim3(256), 0, st, s.partial, s.zpart,
+                     s.tiles * s.nz, s.tiles, out, out + POL_NSTAT, pop);
   return hipGetLastError();
 }
 
 template <typename S>
-static void launch_pop(const StepArgs& a, double* out_dev, dim3 grid, hipStream_t st) {
+static void launch_pop(const StepArgs& a, unsigned long long* out_dev, dim3 grid, hipStream_t st) {
   if (a.records)
     hipLaunchKernelGGL((k_pop_nonfinite<S, true>), grid, dim3(BLOCK), 0, st, a, out_dev);
   else
     hipLaunchKernelGGL((k_pop_nonfinite<S, false>), grid, dim3(BLOCK), 0, st, a, out_dev);
 }
 
-hipError_t launch_pop_nonfinite(int storage, const StepArgs& a, double* out_dev, const Grid& g, hipStream_t st) {
+hipError_t launch_pop_nonfinite(int storage, const StepArgs& a, unsigned long long* out_dev, const Grid& g,
+                                hipStream_t st) {
   const dim3 grid(g.launch);
   switch (storage) {
     case POL_F32: launch_pop<float>(a, out_dev, grid, st); break;

@@ -100,13 +100,16 @@ struct StatsArgs {
   double* partial;        // [nz * tiles][POL_NSTAT]
   double* zpart;          // [nz * tiles]
 };
-// Statistics into out_dev[POL_NSTAT] and the per-plane density sums into
-// zout_dev[nz] (device), deterministic block order.
-hipError_t launch_field_stats(bool real_double, const StatsArgs& s, double* out_dev, double* zout_dev, hipStream_t st);
-// NaN / Inf populations of a.fin over the non-solid cells of the launch list,
-// added to out_dev[POL_STAT_FLUID_POP_NAN], [POL_STAT_FLUID_POP_INF] (zero
-// after launch_field_stats).
-hipError_t launch_pop_nonfinite(int storage, const StepArgs& a, double* out_dev, const Grid& g, hipStream_t st);
+// Block partials of the statistics and of the per-plane density sums.
+hipError_t launch_field_stats(bool real_double, const StatsArgs& s, hipStream_t st);
+// {NaN, Inf} populations of a.fin over the non-solid cells of the launch list,
+// added to out_dev[2].
+hipError_t launch_pop_nonfinite(int storage, const StepArgs& a, unsigned long long* out_dev, const Grid& g,
+                                hipStream_t st);
+// Fold of the partials in a fixed order: the statistics into out[POL_NSTAT]
+// (pinned host memory) and with profile the plane sums into the nz values
+// after them; pop (or null): the counts of launch_pop_nonfinite, zeroed.
+hipError_t launch_stats_final(const StatsArgs& s, bool profile, double* out, unsigned long long* pop, hipStream_t st);
 // Emergency stabilisation of rho / u and of the populations in a.fout.
 hipError_t launch_stabilize(int storage, const StepArgs& a, float max_u, float min_rho, float max_rho, const Grid& g,
                             hipStream_t st);

@@ -46,3 +46,29 @@ def test_counts_without_flags(shape):
     ctx.f_current[18, -1] = float("-inf")
     s, _ = D.field_statistics(ctx, populations=True)
     assert s["fluid_pop_nan"] == 1 and s["fluid_pop_inf"] == 1
+
+
+def test_calls_with_and_without_the_scan():
+    """The scan's counts belong to the call that asks for them, and the other
+    statistics and the plane profile do not depend on it."""
+    wl = WL.v60_config(33, "f32")
+    ctx = HipContext(wl.config, wl.geometry.flags)
+    ctx.init_equilibrium()
+    ctx.step(3, L.POL_WANT_MACRO)
+    clean = ctx.f_current.clone()
+    at = int(ctx.layout.run_slots[len(ctx.layout.run_slots) // 2])
+    while wl.geometry.kind.reshape(-1)[ctx.layout.slot_dense[at]] == L.POL_KIND_SOLID:
+        at += 1
+    want, profile = D.field_statistics(ctx)
+    for planted in (3, 0, 5):
+        ctx.f_current.copy_(clean)
+        ctx.f_current.view(19, -1)[:planted, at] = float("nan")
+        s, z = D.field_statistics(ctx, populations=True)
+        assert s["fluid_pop_nan"] == planted and s["fluid_pop_inf"] == 0
+        plain, z2 = D.field_statistics(ctx)
+        assert plain["fluid_pop_nan"] == 0 and plain["fluid_pop_inf"] == 0
+        for key in want:
+            if not key.startswith("fluid_pop"):
+                assert s[key] == plain[key] == want[key], key
+        if profile is not None:
+            assert np.array_equal(z, profile) and np.array_equal(z2, profile)
