@@ -854,8 +854,10 @@ int pol_step_record(pol_ctx* c, void* states, uint64_t stride_bytes, int count, 
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipSetDevice(c->d.device);
   int held = 0;  // fluxes in the pinned buffer
+  const bool outlets = (c->d.options & POL_USE_FLAGS) && c->b.cell_flags;  // no flags: no outlet cell, flux zero
+  for (int i = flux_first; i < count && !outlets; ++i) flux_out[i - flux_first] = 0.0;
   for (int i = 0; i < count && e == hipSuccess; ++i) {
-    const bool flux = i >= flux_first;
+    const bool flux = i >= flux_first && outlets;
     const StepArgs a = make_args(c, (const char*)states + (uint64_t)i * stride_bytes,
                                  i + 1 < count ? (char*)states + (uint64_t)(i + 1) * stride_bytes : final_state,
                                  flux ? WANT_FLUX : 0u);
