@@ -423,7 +423,9 @@ int pol_step_chain(pol_ctx *ctx, void *states, uint64_t stride_bytes, int count,
  * the forward states of the adjoint.  The steps i >= flux_first also give
  * their outlet mass flux (POL_RED_OUTFLUX, FP64) in flux_out[i - flux_first]
  * (host; NULL when flux_first >= count); with any, the call waits for the
- * stream once, at the end (and every 43 + nz fluxes). */
+ * stream once, at the end (and every 43 + nz fluxes).  POL_ERR_INVALID where a
+ * state would lie over the one it is made from: states less than one state
+ * (19 population planes) apart, final_state over the last recorded state. */
 int pol_step_record(pol_ctx *ctx, void *states, uint64_t stride_bytes, int count, void *final_state, int flux_first,
                     double *flux_out, void *stream);
 /* Zero the adjoint state, grad_perm and the inlet-velocity gradient. */

@@ -849,7 +849,14 @@ int pol_step_record(pol_ctx* c, void* states, uint64_t stride_bytes, int count, 
   if (!c || !states || !final_state || count < 1 || flux_first < 0) return POL_ERR_INVALID;
   if (!c->bound) return fail(c, POL_ERR_STATE, "pol_step_record: buffers not bound");
   if (les_fd(c)) return fail(c, POL_ERR_UNSUPPORTED, "pol_step_record: not with the finite-difference LES");
-  if (count > 1 && stride_bytes == 0) return fail(c, POL_ERR_INVALID, "pol_step_record: zero state stride");
+  // a step reads neighbours that other blocks would already have overwritten:
+  // no state may lie over the one it is made from
+  const int64_t state = (int64_t)POL_Q * c->P * (int64_t)storage_bytes(c->d.storage);
+  auto overlap = [&](int64_t apart) { return apart < state && apart > -state; };
+  if (count > 1 && overlap((int64_t)stride_bytes))
+    return fail(c, POL_ERR_INVALID, "pol_step_record: states closer than one state");
+  if (overlap((int64_t)((uintptr_t)final_state - ((uintptr_t)states + (uint64_t)(count - 1) * stride_bytes))))
+    return fail(c, POL_ERR_INVALID, "pol_step_record: final_state overlaps the last recorded state");
   if (flux_first < count && !flux_out) return fail(c, POL_ERR_INVALID, "pol_step_record: flux_out is NULL");
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipSetDevice(c->d.device);
