@@ -64,6 +64,13 @@ static int hip_fail(pol_ctx* c, hipError_t e, const char* where) {
   return fail(c, POL_ERR_HIP, std::string(where) + ": " + hipGetErrorName(e) + " (" + hipGetErrorString(e) + ")");
 }
 
+// The same where work already queued may still write the context's pinned
+// buffer, which a next call on another stream would read.
+static int hip_fail_queued(pol_ctx* c, hipError_t e, const char* where, hipStream_t s) {
+  (void)hipStreamSynchronize(s);
+  return hip_fail(c, e, where);
+}
+
 static size_t storage_bytes(int s) {
   switch (s) {
     case POL_F32: return 4;
@@ -877,7 +884,7 @@ int pol_step_record(pol_ctx* c, void* states, uint64_t stride_bytes, int count, 
       held = 0;
     }
   }
-  return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_step_record");
+  return e == hipSuccess ? POL_OK : hip_fail_queued(c, e, "pol_step_record", s);
 }
 
 int pol_adjoint_collect(pol_ctx* c, double* out4, void* stream) {
@@ -1305,7 +1312,8 @@ static int thermal_step(pol_ctx* c, int nsteps, const void* velocity, int32_t* u
       if (e == hipSuccess) *unstable_out = (int32_t)*v;
     }
   }
-  return e == hipSuccess ? POL_OK : hip_fail(c, e, "pol_thermal_step");
+  if (e == hipSuccess) return POL_OK;
+  return stats4 || unstable_out ? hip_fail_queued(c, e, "pol_thermal_step", s) : hip_fail(c, e, "pol_thermal_step");
 }
 
 int pol_thermal_step(pol_ctx* c, int nsteps, int32_t* unstable_out, void* stream) {

@@ -42,3 +42,7 @@ def _run(abi, tmp_path, name):
 
 def test_step_record_refuses_overlapping_states(abi, tmp_path):
     _run(abi, tmp_path, "step_record")
+
+
+def test_a_failed_launch_leaves_nothing_queued(abi, tmp_path):
+    _run(abi, tmp_path, "failed_launch")
