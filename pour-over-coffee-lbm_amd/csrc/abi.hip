@@ -41,6 +41,9 @@ struct pol_ctx {
   double* stat_partial = nullptr;   // [nz * stat_tiles][POL_NSTAT]
   double* stat_zpart = nullptr;     // [nz * stat_tiles]
   unsigned long long* pop_dev = nullptr;  // [2] NaN, Inf populations of the scan (zero between calls)
+  // pop_dev, bad_dev[1] hold the counts of a call that failed before the fold
+  // that takes and clears them: the next call that counts clears them first
+  bool pop_left = false, fast_left = false;
   // multiphase phase field
   bool mp = false;
   pol_multiphase_desc md{};
@@ -929,11 +932,14 @@ int pol_field_stats(pol_ctx* c, const pol_stats_opts* o, double* out, double* z_
   if (e == hipSuccess) e = launch_field_stats(d.storage == POL_F64, s, st);
   if (e == hipSuccess && o->with_populations) {
     const StepArgs a = make_args(c, c->b.f[c->cur], nullptr, 0u);
-    e = launch_pop_nonfinite(d.storage, a, c->pop_dev, c->wgrid, st);
+    if (c->pop_left) e = launch_zero_real(true, c->pop_dev, 2, st);
+    c->pop_left = true;
+    if (e == hipSuccess) e = launch_pop_nonfinite(d.storage, a, c->pop_dev, c->wgrid, st);
   }
   if (e == hipSuccess) e = launch_stats_final(s, z_profile != nullptr, c->host, o->with_populations ? c->pop_dev : nullptr, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
-  if (e != hipSuccess) return hip_fail(c, e, "pol_field_stats");
+  if (e != hipSuccess) return hip_fail_queued(c, e, "pol_field_stats", st);
+  if (o->with_populations) c->pop_left = false;
   std::memcpy(out, c->host, POL_NSTAT * sizeof(double));
   if (z_profile) std::memcpy(z_profile, c->host + POL_NSTAT, (size_t)d.nz * sizeof(double));
   return POL_OK;
@@ -1293,12 +1299,17 @@ static int thermal_step(pol_ctx* c, int nsteps, const void* velocity, int32_t* u
   ThermalArgs a = thermal_args(c);
   a.u_src = velocity;
   a.report = stats4 ? 1u : 0u;
+  if (stats4) {
+    if (e == hipSuccess && c->fast_left) e = launch_zero_real(false, c->bad_dev, 2, s);
+    c->fast_left = true;
+  }
   if (e == hipSuccess)
     e = launch_thermal_steps(c->d.storage == POL_F64, a, c->tb.g, c->tb.temperature, c->gcur, c->tcur,
                              nsteps, c->partial, c->host, s);
   if (e == hipSuccess && stats4) {
     e = hipStreamSynchronize(s);
     if (e == hipSuccess) {
+      c->fast_left = false;
       std::memcpy(stats4, c->host, 4 * sizeof(double));
       if (unstable_out) *unstable_out = (int32_t)c->host[4];
     }

@@ -67,6 +67,9 @@ hipError_t launch_reduce_final(double*, uint32_t, double* out, hipStream_t) {
 hipError_t launch_flux_fold(const double*, uint32_t, double* out, hipStream_t) {
   return launch([=] { *out = 0.5; });
 }
+hipError_t launch_zero_real(bool dbl, void* p, size_t n, hipStream_t) {
+  return launch([=] { memset(p, 0, n * (dbl ? 8 : 4)); });
+}
 }  // namespace pol
 
 #define CHECK(x)                                                   \

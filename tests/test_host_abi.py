@@ -46,3 +46,7 @@ def test_step_record_refuses_overlapping_states(abi, tmp_path):
 
 def test_a_failed_launch_leaves_nothing_queued(abi, tmp_path):
     _run(abi, tmp_path, "failed_launch")
+
+
+def test_counts_start_from_zero_after_a_failed_call(abi, tmp_path):
+    _run(abi, tmp_path, "counts")
