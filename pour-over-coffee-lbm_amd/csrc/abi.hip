@@ -354,7 +354,7 @@ static StepArgs make_args(const pol_ctx* c, const void* fin, void* fout, uint32_
   a.per_xcd = c->wgrid.per_xcd;
   a.nblk = c->wgrid.nblk;
   a.options = d.options;
-  a.what = what;
+  a.what = what & (POL_WANT_MACRO | POL_WANT_REDUCE);  // a caller's other bits mean nothing (WANT_FLUX is one)
   a.tau0 = d.tau;
   a.nu0 = (d.tau - 0.5) / 3.0;
   a.les_c = 18.0 * std::sqrt(2.0) * d.cs_smag * d.cs_smag;
@@ -875,9 +875,9 @@ int pol_step_record(pol_ctx* c, void* states, uint64_t stride_bytes, int count, 
   for (int i = flux_first; i < count && !outlets; ++i) flux_out[i - flux_first] = 0.0;
   for (int i = 0; i < count && e == hipSuccess; ++i) {
     const bool flux = i >= flux_first && outlets;
-    const StepArgs a = make_args(c, (const char*)states + (uint64_t)i * stride_bytes,
-                                 i + 1 < count ? (char*)states + (uint64_t)(i + 1) * stride_bytes : final_state,
-                                 flux ? WANT_FLUX : 0u);
+    StepArgs a = make_args(c, (const char*)states + (uint64_t)i * stride_bytes,
+                           i + 1 < count ? (char*)states + (uint64_t)(i + 1) * stride_bytes : final_state, 0u);
+    if (flux) a.what = WANT_FLUX;
     e = launch_stream_collide(c->d.storage, a, true, c->wgrid, s);
     if (e != hipSuccess || !flux) continue;
     e = launch_flux_fold(c->partial, c->wgrid.nblk, c->host + held++, s);

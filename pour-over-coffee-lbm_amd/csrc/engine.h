@@ -65,7 +65,8 @@ struct LesFdArgs {
 hipError_t launch_les_fd(bool dbl, const LesFdArgs& a, hipStream_t s);
 
 // StepArgs::what bit beside POL_WANT_*: the step's outlet mass flux
-// (POL_RED_OUTFLUX) per block into partial[block].
+// (POL_RED_OUTFLUX) per block into partial[block].  Not a bit of the ABI, and
+// not together with POL_WANT_REDUCE, whose rows lie in the same buffer.
 constexpr uint32_t WANT_FLUX = 0x80000000u;
 // Fold those partials into out[0] (device or pinned host memory), in a fixed order.
 hipError_t launch_flux_fold(const double* partial, uint32_t nblk, double* out, hipStream_t s);

@@ -2,7 +2,6 @@
 // fold that takes the counts: the next call counts from zero.
 #include "stubs.h"
 
-
 namespace pol {
 hipError_t launch_field_stats(bool, const StatsArgs&, hipStream_t) { return launch([] {}); }
 hipError_t launch_pop_nonfinite(int, const StepArgs&, unsigned long long* out, const Grid&, hipStream_t) {
@@ -41,14 +40,6 @@ int main() {
   Box box;
   pol_stats_opts o{};
   o.with_populations = 1;
-  std::vector<float> fields(4 * Box::cells);
-  pol_buffers b{};
-  b.f[0] = box.at(0);
-  b.f[1] = box.at(1);
-  b.cell_flags = box.flags.data();
-  b.rho = fields.data();
-  b.u = fields.data() + Box::cells;
-  CHECK(pol_bind(box.c, &b) == POL_OK);
   double out[POL_NSTAT];
   auto counts = [&](int nan, int inf) {
     CHECK(pol_field_stats(box.c, &o, out, nullptr, nullptr) == POL_OK);

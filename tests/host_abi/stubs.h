@@ -88,17 +88,20 @@ struct Box {
   std::vector<uint32_t> flags = std::vector<uint32_t>(cells);
   pol_ctx* c = nullptr;
   char* at(double states) { return mem.data() + (size_t)(states * state_bytes); }
-  Box() {
+  explicit Box(uint32_t options = 0) {
     pol_desc d{};
     d.nx = nx; d.ny = ny; d.nz = nz;
     d.storage = POL_F32;
-    d.options = POL_USE_FLAGS;
+    d.options = POL_USE_FLAGS | options;
     d.tau = 0.6;
     CHECK(pol_create(&c, &d) == POL_OK);
     pol_buffers b{};
     b.f[0] = at(0);
     b.f[1] = at(1);
     b.cell_flags = flags.data();
+    b.force = at(13);
+    b.rho = at(14);
+    b.u = at(14.5);
     CHECK(pol_bind(c, &b) == POL_OK);
   }
   ~Box() { pol_destroy(c); }

@@ -50,3 +50,7 @@ def test_a_failed_launch_leaves_nothing_queued(abi, tmp_path):
 
 def test_counts_start_from_zero_after_a_failed_call(abi, tmp_path):
     _run(abi, tmp_path, "counts")
+
+
+def test_undefined_bits_of_what_do_nothing(abi, tmp_path):
+    _run(abi, tmp_path, "what_bits")
