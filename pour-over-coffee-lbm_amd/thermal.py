@@ -361,6 +361,16 @@ class ThermalLBM:
             self._hs.copy_(src)
 
 
+# The methods whose work the coupled step may do in one native call.  A caller's
+# thermal solver that has its own version of one (a subclass, a replaced
+# method, another class) gets it called instead.
+_FUSED = {name: vars(ThermalLBM)[name] for name in ("set_velocity_field", "step", "get_temperature_stats", "compute_diagnostics")}
+
+
+def _has_own(thermal_solver, *names: str) -> bool:
+    return any(getattr(getattr(thermal_solver, n, None), "__func__", None) is not _FUSED[n] for n in names)
+
+
 @dataclass
 class CouplingConfig:
     """thermal_fluid_coupled.py:35-42."""
@@ -439,24 +449,27 @@ class ThermalFluidCoupledSolver:
         self.fluid_solver.step()
         t1 = time.time()
         self.performance_stats["fluid_time"] += t1 - t0
+        ts = self.thermal_solver
         velocity = None  # handed over inside the first sub-cycle
         if self.coupling_step % cfg.coupling_frequency == 0:
             get = getattr(self.fluid_solver, "get_velocity_field_for_thermal_coupling", None)
             velocity = get() if get is not None else self.fluid_solver.u
-            if cfg.thermal_subcycles < 1:
-                self.thermal_solver.set_velocity_field(velocity)
+            if cfg.thermal_subcycles < 1 or _has_own(ts, "set_velocity_field", "step"):
+                ts.set_velocity_field(velocity)
+                velocity = None
             self.performance_stats["coupling_time"] += time.time() - t1
         t2 = time.time()
         if not self.fused_reset:
-            self.thermal_solver.reset_heat_source_to_base(self.base_heat_source)
+            ts.reset_heat_source_to_base(self.base_heat_source)
         figures = None  # of the check below, where a step forms them itself
         for k in range(cfg.thermal_subcycles):
             if k == 0 and velocity is not None:
-                if cfg.enable_diagnostics and cfg.thermal_subcycles == 1:
+                if cfg.enable_diagnostics and cfg.thermal_subcycles == 1 and not _has_own(
+                        ts, "get_temperature_stats", "compute_diagnostics"):
                     figures = np.zeros(4, dtype=np.float64)
-                ok = self.thermal_solver.step_with_velocity(velocity, figures)
+                ok = ts.step_with_velocity(velocity, figures)
             else:
-                ok = self.thermal_solver.step()
+                ok = ts.step()
             if not ok:
                 return False
         self.performance_stats["thermal_time"] += time.time() - t2
@@ -469,15 +482,21 @@ class ThermalFluidCoupledSolver:
     def _check_coupling_stability(self, figures: Optional[np.ndarray] = None) -> bool:
         """thermal_fluid_coupled.py:237-262, its figures from one device pass
         or from the step (`figures`)."""
-        out = figures
-        if out is None:
-            out = np.zeros(4, dtype=np.float64)
-            self.thermal_solver._coupling_stats(out)
-        tmin, tmax, _, fast_cells = (float(v) for v in out)
+        ts = self.thermal_solver
+        if figures is None and _has_own(ts, "get_temperature_stats", "compute_diagnostics"):
+            tmin, tmax, _ = ts.get_temperature_stats()
+            fast_cells = None
+        else:
+            if figures is None:
+                figures = np.zeros(4, dtype=np.float64)
+                ts._coupling_stats(figures)
+            tmin, tmax, _, fast_cells = (float(v) for v in figures)
         if tmax > 150.0 or tmin < -10.0:
             return False
         if abs(tmax - tmin) > self.coupling_config.max_coupling_error:
             return False
+        if fast_cells is None:
+            return not bool((torch.linalg.vector_norm(ts._vel, dim=0) > 1.0).any())
         return fast_cells == 0
 
     def get_coupling_diagnostics(self) -> dict:
