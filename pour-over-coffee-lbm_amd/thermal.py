@@ -450,20 +450,21 @@ class ThermalFluidCoupledSolver:
         t1 = time.time()
         self.performance_stats["fluid_time"] += t1 - t0
         ts = self.thermal_solver
-        velocity = None  # handed over inside the first sub-cycle
+        hand_over = False  # the velocity, inside the first sub-cycle
         if self.coupling_step % cfg.coupling_frequency == 0:
             get = getattr(self.fluid_solver, "get_velocity_field_for_thermal_coupling", None)
             velocity = get() if get is not None else self.fluid_solver.u
             if cfg.thermal_subcycles < 1 or _has_own(ts, "set_velocity_field", "step"):
                 ts.set_velocity_field(velocity)
-                velocity = None
+            else:
+                hand_over = True
             self.performance_stats["coupling_time"] += time.time() - t1
         t2 = time.time()
         if not self.fused_reset:
             ts.reset_heat_source_to_base(self.base_heat_source)
         figures = None  # of the check below, where a step forms them itself
         for k in range(cfg.thermal_subcycles):
-            if k == 0 and velocity is not None:
+            if k == 0 and hand_over:
                 if cfg.enable_diagnostics and cfg.thermal_subcycles == 1 and not _has_own(
                         ts, "get_temperature_stats", "compute_diagnostics"):
                     figures = np.zeros(4, dtype=np.float64)

@@ -168,3 +168,11 @@ def test_an_object_with_the_documented_methods_only(monkeypatch, subcycles):
     s = _coupled(monkeypatch, calls, Plain(), thermal_subcycles=subcycles)
     assert s.step()
     assert calls == ["fluid", "velocity"] + ["reset"] * (subcycles != 1) + ["step"] * subcycles + ["statistics"]
+
+
+def test_no_velocity_is_refused(monkeypatch):
+    calls = []
+    s = _coupled(monkeypatch, calls, _thermal(calls))
+    s.fluid_solver.u = None
+    with pytest.raises(TypeError):
+        s.step()
