@@ -462,11 +462,13 @@ class ThermalFluidCoupledSolver:
         t2 = time.time()
         if not self.fused_reset:
             ts.reset_heat_source_to_base(self.base_heat_source)
-        figures = None  # of the check below, where a step forms them itself
+        # the figures of the check below, where a step forms them itself
+        figures = None
+        own_check = getattr(self._check_coupling_stability, "__func__", None) is not _COUPLING_CHECK
         for k in range(cfg.thermal_subcycles):
             if k == 0 and hand_over:
-                if cfg.enable_diagnostics and cfg.thermal_subcycles == 1 and not _has_own(
-                        ts, "get_temperature_stats", "compute_diagnostics"):
+                if cfg.enable_diagnostics and cfg.thermal_subcycles == 1 and not (
+                        own_check or _has_own(ts, "get_temperature_stats", "compute_diagnostics")):
                     figures = np.zeros(4, dtype=np.float64)
                 ok = ts.step_with_velocity(velocity, figures)
             else:
@@ -474,7 +476,8 @@ class ThermalFluidCoupledSolver:
             if not ok:
                 return False
         self.performance_stats["thermal_time"] += time.time() - t2
-        if cfg.enable_diagnostics and not self._check_coupling_stability(figures):
+        if cfg.enable_diagnostics and not (self._check_coupling_stability() if figures is None
+                                           else self._check_coupling_stability(figures)):
             return False
         self.coupling_step += 1
         self.performance_stats["total_steps"] += 1
@@ -552,3 +555,6 @@ class ThermalFluidCoupledSolver:
 
     def get_temperature_field(self):
         return self.thermal_solver.temperature
+
+
+_COUPLING_CHECK = ThermalFluidCoupledSolver._check_coupling_stability  # a caller's own takes no figures

@@ -176,3 +176,26 @@ def test_no_velocity_is_refused(monkeypatch):
     s.fluid_solver.u = None
     with pytest.raises(TypeError):
         s.step()
+
+
+@pytest.mark.parametrize("subcycles", [0, 1, 2])
+@pytest.mark.parametrize("mode", MODES)
+def test_an_own_stability_check_takes_no_argument(monkeypatch, mode, subcycles):
+    """_check_coupling_stability is the reference's own name (thermal_fluid_coupled.py:237)."""
+    calls, answer = [], [True]
+
+    def check(self):
+        calls.append("own check")
+        return answer[0]
+
+    cls = TH.ThermalFluidCoupledSolver
+    if mode == "subclass":
+        monkeypatch.setattr(TH, "ThermalFluidCoupledSolver", type("Own", (cls,), {"_check_coupling_stability": check}))
+    elif mode == "class":
+        monkeypatch.setattr(cls, "_check_coupling_stability", check)
+    s = _coupled(monkeypatch, calls, _thermal(calls), thermal_subcycles=subcycles)
+    if mode == "object":
+        monkeypatch.setattr(s, "_check_coupling_stability", check.__get__(s))
+    assert s.step() and calls[-1] == "own check" and calls.count("own check") == 1
+    answer[0] = False
+    assert not s.step()
