@@ -145,12 +145,13 @@ class AdjointProblem:
         store, the last into the context's next buffer, in one native call;
         the sum of their objective steps' outlet fluxes."""
         ctx, K = self.ctx, self.checkpoint
-        first = max(0, min(K, (self.steps - self.window) - start))  # first objective step of these
+        objective = [i for i in range(K) if self.objective_step(start + i)]
+        first = objective[0] if objective else K
         flux = np.zeros(max(K - first, 1), dtype=np.float64)
         stride = self.seg[0].numel() * self.seg.element_size()
         L.check(ctx.lib.pol_step_record(ctx.handle, L.ptr(self.seg), stride, K, L.ptr(ctx.f_next), first,
                                         flux.ctypes.data, L.stream_handle()), ctx.handle, "pol_step_record")
-        return sum(flux.tolist(), 0.0)
+        return sum((float(flux[i - first]) for i in objective), 0.0)
 
     def forward_time(self) -> float:
         """Seconds for the plain forward run (no reductions, no checkpoints)."""
