@@ -561,7 +561,9 @@ int pol_thermal_step(pol_ctx *ctx, int nsteps, int32_t *unstable_out, void *stre
  * velocity (real [3][cells]) into the bound velocity buffer: the first step
  * reads it from there and stores it (the coupled loop's hand-over of the fluid
  * velocity, thermal_fluid_coupled.py:183-190, without a pass of its own).  The
- * bound velocity buffer is written.  With stats4 != NULL it receives what
+ * bound velocity buffer is written; velocity may be that buffer itself, but
+ * POL_ERR_INVALID where it lies across it, the heat source or the population
+ * buffer that the first step writes.  With stats4 != NULL it receives what
  * pol_thermal_coupling_stats would return after the steps, formed inside them;
  * synchronous then. */
 int pol_thermal_step_with_velocity(pol_ctx *ctx, int nsteps, const void *velocity, int32_t *unstable_out,

@@ -1339,6 +1339,15 @@ int pol_thermal_step_with_velocity(pol_ctx* c, int nsteps, const void* velocity,
   if (!c->thermal) return fail(c, POL_ERR_STATE, "pol_thermal_step_with_velocity: thermal buffers not bound");
   if (!(c->td.options & POL_THERMAL_CONVECTION))
     return fail(c, POL_ERR_STATE, "pol_thermal_step_with_velocity: needs POL_THERMAL_CONVECTION");
+  // the first step reads the velocity while it writes its own buffer of it, the
+  // populations and the sources: it may be that buffer, but not lie across any
+  const uintptr_t plane = (uintptr_t)c->N * (c->d.storage == POL_F64 ? 8 : 4), v = (uintptr_t)velocity;
+  auto across = [&](const void* p, uintptr_t planes) {
+    return v < (uintptr_t)p + planes * plane && (uintptr_t)p < v + 3 * plane;
+  };
+  if ((velocity != c->tb.velocity && across(c->tb.velocity, 3)) || across(c->tb.g[1 - c->gcur], 7) ||
+      across(c->tb.heat_source, 1))
+    return fail(c, POL_ERR_INVALID, "pol_thermal_step_with_velocity: velocity overlaps a buffer that the step writes");
   return thermal_step(c, nsteps, velocity, unstable_out, stats4, stream);
 }
 

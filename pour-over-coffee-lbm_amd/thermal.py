@@ -205,7 +205,11 @@ class ThermalLBM:
         v = self._vel
         if (self.is_initialized and self.enable_convection and isinstance(src, torch.Tensor) and src.device == v.device
                 and src.dtype == v.dtype and src.shape == v.shape and src.is_contiguous()):
-            return self._step(src, stats)
+            try:
+                return self._step(src, stats)
+            except L.PolError as e:
+                if e.status != L.POL_ERR_INVALID:
+                    raise  # else: it lies across a buffer that the step writes, and is copied first
         self.set_velocity_field(src)
         ok = self._step(None)
         if ok and stats is not None:

@@ -54,3 +54,7 @@ def test_counts_start_from_zero_after_a_failed_call(abi, tmp_path):
 
 def test_undefined_bits_of_what_do_nothing(abi, tmp_path):
     _run(abi, tmp_path, "what_bits")
+
+
+def test_velocity_across_a_written_buffer_is_refused(abi, tmp_path):
+    _run(abi, tmp_path, "thermal_velocity")

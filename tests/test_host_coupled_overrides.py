@@ -199,3 +199,16 @@ def test_an_own_stability_check_takes_no_argument(monkeypatch, mode, subcycles):
     assert s.step() and calls[-1] == "own check" and calls.count("own check") == 1
     answer[0] = False
     assert not s.step()
+
+
+def test_a_velocity_that_the_step_would_overwrite_is_copied_first(monkeypatch):
+    calls = []
+    th = _thermal(calls)
+    s = _coupled(monkeypatch, calls, th)
+    lib = th.lib
+    th.lib = type("Refuses", (), {
+        "pol_thermal_step_with_velocity": staticmethod(lambda *a: TH.L.POL_ERR_INVALID),
+        "__getattr__": lambda self, name: getattr(lib, name)})()
+    assert s.step()
+    assert torch.equal(th._vel, torch.full_like(th._vel, 0.25))
+    assert calls == ["fluid", "pol_thermal_step", "pol_thermal_coupling_stats"]
