@@ -217,12 +217,23 @@ inline uint32_t launch_blocks(uint32_t order, const Grid& g) {
 // eight L2s and the planes above and below are fetched again by other XCDs.
 // A pass whose fields stay in the last-level cache gives each XCD one range
 // of planes; one that streams from HBM keeps one front, in groups of 16
-// blocks (4096 cells) per XCD.  Measured, linear / ranges / groups of 16 (us):
+// blocks (4096 cells) per XCD.  Kernel times, linear / ranges / groups of 16
+// (us, FP32; convection: the collide and the temperature pass of a step):
 //                           phase step            eddy viscosity        convection step
-//   64^3                    7.8 / 8.0 / 7.7       6.9 / 7.0 / 6.8       8.6 / 10.3 / 10.6
-//   128^3                   14.9 / 12.9 / 14.5    14.0 / 11.2 / 12.5    39.0 / 37.2 / 38.1
-//   160^3                   28.6 / 21.7 / 27.9    28.5 / 19.9 / 27.2    76.7 / 73.9 / 74.8
+//   64^3                    4.1 / 4.0 / 4.3       3.2 / 3.2 / 3.2       8.0 / 9.8 / 9.8
+//   80^3                    5.7 / 5.1 / 5.7       4.0 / 4.0 / 4.0       12.4 / 13.1 / 13.7
+//   96^3                    8.2 / 7.5 / 8.3       5.4 / 5.2 / 5.4       18.6 / 19.2 / 19.7
+//   104^3                                                               23.7 / 22.0 / 23.1
+//   128^3                   14.6 / 12.9 / 14.7    12.1 / 9.1 / 10.0     43.5 / 37.5 / 38.4
+//   144^3                   21.9 / 16.7 / 21.2    16.9 / 12.4 / 17.1    53.3 / 49.9 / 52.5
+//   200^3                   62.2 / 54.6 / 54.5    59.5 / 26.4 / 42.5    collide 103.6 / 96.3 / 98.0
+//   210^3                   74.2 / 64.2 / 62.6    72.1 / 30.2 / 49.4    collide 130.6 / 130.9 / 120.5
 //   224^3                   80.1 / 85.8 / 75.4    82.8 / 64.1 / 63.8    228.9 / 236.6 / 222.2
+// A convection step's temperature pass takes the blocks in linear order, so
+// ranges cost it the populations that the collide pass has just left in the
+// same XCD's L2; that outweighs the neighbours below about 70 MiB (FP32 96^3,
+// 68 MiB, above; 181 x 97 x 53, 71 MiB, 21.2 / 20.0 us; FP64 72^3, 57 MiB,
+// 14.9 / 16.5, and 80^3, 78 MiB, 21.8 / 20.4), where it stays linear.
 // (The pressure drive over the cup is 15-25 % slower in ranges, whose cells
 // are unevenly solid, and within 4 % in groups: it stays linear, as do passes
 // without neighbours.)
@@ -234,8 +245,10 @@ inline BlockOrder linear_order(uint64_t cells) {
   const Grid g = make_grid(cells);
   return BlockOrder{ORDER_LINEAR, g.per_xcd, g.nblk};
 }
-// bytes: what the pass reads and writes
-inline BlockOrder stencil_order(uint64_t cells, uint64_t bytes) {
+constexpr uint64_t CONVECTION_LINEAR_BYTES = 70ull << 20;
+// bytes: what the pass reads and writes; below linear_bytes it stays linear
+inline BlockOrder stencil_order(uint64_t cells, uint64_t bytes, uint64_t linear_bytes = 0) {
+  if (bytes < linear_bytes) return linear_order(cells);
   const Grid g = make_grid(cells);
   return BlockOrder{bytes <= LAST_LEVEL_BYTES ? ORDER_XCD_RANGES : 4u, g.per_xcd, g.nblk};
 }

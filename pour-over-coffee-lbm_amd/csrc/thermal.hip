@@ -467,8 +467,8 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
   // boundary value rather than sum g).
   // convection reads the temperature's neighbours (populations, T, u and the
   // sources, 80 B a cell); pure diffusion reads only the cell's own values
-  const BlockOrder ord =
-      base.conv ? stencil_order(base.N, 20ull * sizeof(R) * base.N) : linear_order(base.N);
+  const BlockOrder ord = base.conv ? stencil_order(base.N, 20ull * sizeof(R) * base.N, CONVECTION_LINEAR_BYTES)
+                                   : linear_order(base.N);
   const dim3 cgrid(launch_blocks(ord));
   const bool nt = 2ull * TQ * sizeof(R) * base.N > LAST_LEVEL_BYTES;  // both population buffers
   for (int n = 0; n < nsteps; ++n) {
