@@ -368,11 +368,22 @@ class ThermalLBM:
 # The methods whose work the coupled step may do in one native call.  A caller's
 # thermal solver that has its own version of one (a subclass, a replaced
 # method, another class) gets it called instead.
-_FUSED = {name: vars(ThermalLBM)[name] for name in ("set_velocity_field", "step", "get_temperature_stats", "compute_diagnostics")}
+_STEP, _SET_VELOCITY = ThermalLBM.step, ThermalLBM.set_velocity_field
+_STATS, _DIAGNOSTICS = ThermalLBM.get_temperature_stats, ThermalLBM.compute_diagnostics
 
 
-def _has_own(thermal_solver, *names: str) -> bool:
-    return any(getattr(getattr(thermal_solver, n, None), "__func__", None) is not _FUSED[n] for n in names)
+def _own_step(ts) -> bool:
+    try:
+        return ts.step.__func__ is not _STEP or ts.set_velocity_field.__func__ is not _SET_VELOCITY
+    except AttributeError:  # no bound method
+        return True
+
+
+def _own_statistics(ts) -> bool:
+    try:
+        return ts.get_temperature_stats.__func__ is not _STATS or ts.compute_diagnostics.__func__ is not _DIAGNOSTICS
+    except AttributeError:
+        return True
 
 
 @dataclass
@@ -458,7 +469,7 @@ class ThermalFluidCoupledSolver:
         if self.coupling_step % cfg.coupling_frequency == 0:
             get = getattr(self.fluid_solver, "get_velocity_field_for_thermal_coupling", None)
             velocity = get() if get is not None else self.fluid_solver.u
-            if cfg.thermal_subcycles < 1 or _has_own(ts, "set_velocity_field", "step"):
+            if cfg.thermal_subcycles < 1 or _own_step(ts):
                 ts.set_velocity_field(velocity)
             else:
                 hand_over = True
@@ -466,13 +477,11 @@ class ThermalFluidCoupledSolver:
         t2 = time.time()
         if not self.fused_reset:
             ts.reset_heat_source_to_base(self.base_heat_source)
-        # the figures of the check below, where a step forms them itself
-        figures = None
-        own_check = getattr(self._check_coupling_stability, "__func__", None) is not _COUPLING_CHECK
+        figures = None  # of the check below, where a step forms them itself
         for k in range(cfg.thermal_subcycles):
             if k == 0 and hand_over:
                 if cfg.enable_diagnostics and cfg.thermal_subcycles == 1 and not (
-                        own_check or _has_own(ts, "get_temperature_stats", "compute_diagnostics")):
+                        self._own_check() or _own_statistics(ts)):
                     figures = np.zeros(4, dtype=np.float64)
                 ok = ts.step_with_velocity(velocity, figures)
             else:
@@ -487,18 +496,21 @@ class ThermalFluidCoupledSolver:
         self.performance_stats["total_steps"] += 1
         return True
 
+    def _own_check(self) -> bool:
+        return getattr(self._check_coupling_stability, "__func__", None) is not _COUPLING_CHECK
+
     def _check_coupling_stability(self, figures: Optional[np.ndarray] = None) -> bool:
         """thermal_fluid_coupled.py:237-262, its figures from one device pass
         or from the step (`figures`)."""
         ts = self.thermal_solver
-        if figures is None and _has_own(ts, "get_temperature_stats", "compute_diagnostics"):
+        if figures is None and _own_statistics(ts):
             tmin, tmax, _ = ts.get_temperature_stats()
             fast_cells = None
         else:
             if figures is None:
                 figures = np.zeros(4, dtype=np.float64)
                 ts._coupling_stats(figures)
-            tmin, tmax, _, fast_cells = (float(v) for v in figures)
+            tmin, tmax, _, fast_cells = figures.tolist()
         if tmax > 150.0 or tmin < -10.0:
             return False
         if abs(tmax - tmin) > self.coupling_config.max_coupling_error:
