@@ -41,9 +41,11 @@ struct pol_ctx {
   double* stat_partial = nullptr;   // [nz * stat_tiles][POL_NSTAT]
   double* stat_zpart = nullptr;     // [nz * stat_tiles]
   unsigned long long* pop_dev = nullptr;  // [2] NaN, Inf populations of the scan (zero between calls)
-  // pop_dev, bad_dev[1] hold the counts of a call that failed before the fold
-  // that takes and clears them: the next call that counts clears them first
-  bool pop_left = false, fast_left = false;
+  // pop_dev, bad_dev[1] hold what the allocation held, or the counts of a call
+  // that failed before the fold that takes and clears them: the next call that
+  // counts clears them first (a copy of zeros at creation waits for the
+  // device's queued work, 12 us each on an idle one)
+  bool pop_left = true, fast_left = true;
   // multiphase phase field
   bool mp = false;
   pol_multiphase_desc md{};
@@ -145,8 +147,6 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
   hipError_t e = hipSetDevice(d.device);
   if (e == hipSuccess) e = hipMalloc((void**)&c->partial, (size_t)c->part_cap * POL_NRED * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&c->bad_dev, 2 * sizeof(uint32_t));
-  const uint32_t none[2] = {0u, 0u};
-  if (e == hipSuccess) e = hipMemcpy(c->bad_dev, none, sizeof(none), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc((void**)&c->adj_partial, (size_t)c->part_cap * 4 * sizeof(double));
   // statistics: up to 12 blocks per plane (2688 blocks at 224^3, each lane
   // ~8 groups of four cells: the per-block reduction of the 43 statistics is
@@ -160,8 +160,6 @@ int pol_create(pol_ctx** out, const pol_desc* desc) {
   if (e == hipSuccess) e = hipMalloc((void**)&c->stat_partial, sblk * POL_NSTAT * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&c->stat_zpart, sblk * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void**)&c->pop_dev, 2 * sizeof(unsigned long long));
-  const unsigned long long nopop[2] = {0ull, 0ull};
-  if (e == hipSuccess) e = hipMemcpy(c->pop_dev, nopop, sizeof(nopop), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipHostMalloc((void**)&c->host, ((size_t)POL_NSTAT + d.nz) * sizeof(double));
   if (e != hipSuccess) {
     (void)hipHostFree(c->host);

@@ -16,6 +16,7 @@
 
 inline std::deque<std::function<void()>> queued;  // work of the stream, not yet done
 inline std::vector<pol::StepArgs> steps;          // every stream-collide launch
+inline int blocking_copies = 0;
 inline int fail_after = -1;                       // launches that succeed before one fails (-1: all)
 
 inline hipError_t launch(std::function<void()> work) {
@@ -38,11 +39,17 @@ inline void wait_all() {
 extern "C" {
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipMalloc(void** p, size_t n) { *p = calloc(1, n); return hipSuccess; }
+// device memory comes as it was left
+hipError_t hipMalloc(void** p, size_t n) { *p = memset(malloc(n), 0x5a, n); return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned int) { *p = calloc(1, n); return hipSuccess; }
 hipError_t hipFree(void* p) { wait_all(); free(p); return hipSuccess; }
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
-hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { wait_all(); memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
+  ++blocking_copies;
+  wait_all();
+  memcpy(d, s, n);
+  return hipSuccess;
+}
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
   return launch([=] { memcpy(d, s, n); });
 }

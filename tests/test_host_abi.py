@@ -58,3 +58,7 @@ def test_undefined_bits_of_what_do_nothing(abi, tmp_path):
 
 def test_velocity_across_a_written_buffer_is_refused(abi, tmp_path):
     _run(abi, tmp_path, "thermal_velocity")
+
+
+def test_creating_a_context_waits_for_nothing(abi, tmp_path):
+    _run(abi, tmp_path, "create")
