@@ -318,11 +318,14 @@ static StepArgs make_args(const pol_ctx* c, const void* fin, void* fout, uint32_
   // step by 7 % (FP32 compact), 13 % (FP16) and 8 % (FP64); at 128^3, where
   // the step still caches, they cost 25 %.  Not where the planes of an
   // unlisted dense box are no whole number of 64-byte sectors apart: a wave's
-  // stores then end inside sectors, which streaming sends to HBM as
-  // read-modify-writes, while cached stores of neighbouring blocks meet in
-  // one L2 (FP32 180 x 175 x 179: 228 -> 174 us, 241 x 239 x 243: 573 -> 422,
-  // FP16 187 x 150 x 201: 125 -> 101; planes 64 or 128 bytes off a 256-byte
-  // boundary are up to 5 % faster streamed).
+  // stores then end inside sectors, which streaming sends to HBM one by one,
+  // while cached stores of neighbouring blocks meet in one L2 (FP32 180 x 175 x
+  // 179: 228 -> 174 us, 241 x 239 x 243: 573 -> 422, FP16 187 x 150 x 201: 125
+  // -> 101; planes 64 or 128 bytes off a 256-byte boundary are up to 5 % faster
+  // streamed).  Counters at 180 x 175 x 179, streamed / cached: 505 / 432 MB
+  // fetched, 464 / 431 MB written for 429 MB each way.  From the limit on (20
+  // steps and a report, streamed / cached): FP32 121^3 1297 / 1051 us, 125 x 121
+  // x 119 1486 / 1250; FP64 97^3 1342 / 1147; FP16 155 x 153 x 153 1789 / 1334.
   const bool streams = 2ull * a.n_items * Q * storage_bytes(d.storage) > (256ull << 20);
   const bool whole_sectors = a.chunks || ((uint64_t)c->P * storage_bytes(d.storage)) % 64 == 0;
   a.stream_store = streams && whole_sectors ? 1u : 0u;

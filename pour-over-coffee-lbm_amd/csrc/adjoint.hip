@@ -496,7 +496,7 @@ __global__ void __launch_bounds__(BLOCK) k_adjoint(const AdjointArgs A, const ui
   // slots hold the sums over every step since pol_adjoint_reset and are
   // folded once, in block order, by k_adjoint_final when collected
   // (only inlet and outlet cells contribute: other waves write zeros and skip
-  // the FP64 shuffles)
+  // the FP64 reductions)
   __shared__ double sh[BLOCK / 64][4];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const bool contributes = part[0] != R(0) || part[1] != R(0) || part[2] != R(0) || part[3] != R(0);

@@ -15,7 +15,7 @@
 // Statistics kernel: a grid of (tiles, nz) blocks, block (t, z) looping over
 // a strip of plane z; per-lane FP64 accumulators (integer counters for the
 // counts, integer keys for the extremes of |u|) split between two wave
-// pairs, wave64 shuffles, one partial per block per statistic, folded in
+// pairs, wave64 reductions, one partial per block per statistic, folded in
 // block order by one block per statistic (deterministic).
 // The per-plane density sums of the z profile fall out of the same partials.
 // |u| is formed in FP32 as sqrt((ux*ux + uy*uy) + uz*uz) with explicit

@@ -231,10 +231,13 @@ __device__ inline void store_quad(R* __restrict__ p, uint32_t j, const R (&v)[4]
 // (every wave of a stable state) neither reduces nor stores anything.
 // REP: also the block's {min, max, sum} of T', while they are in registers
 // (a statistics pass over T and u after the step took 0.033 ms at 224^3).
-// NT (populations above the last-level cache): nothing here is read again
-// before the cache has turned over, so loads and stores bypass it (reporting
-// pass at 224^3 85 -> 67 us; cached, its loads also evict what the fluid step
-// that follows would find).
+// NT (populations above the last-level cache): loads and stores bypass it.  In
+// the coupled loop nothing here is read again before the cache has turned over
+// (reporting pass at 224^3 85 -> 67 us; cached, its loads also evict what the
+// fluid step that follows would find).  In a run with convection the next
+// collide pass reads T at once, from HBM then, and the step still gains: what T
+// (45 of 405 MB at 224^3) would keep out of the cache is more (16 steps at
+// 200^3 2586 -> 2284 us, both passes streamed).
 template <typename R, int W, bool REP, bool NT>
 __global__ void __launch_bounds__(256) k_thermal_temperature(const ThermalArgs a, double* __restrict__ partial) {
 #pragma clang fp contract(off)
@@ -470,7 +473,14 @@ static hipError_t thermal_steps(const ThermalArgs& base, void* const g[2], void*
   const BlockOrder ord = base.conv ? stencil_order(base.N, 20ull * sizeof(R) * base.N, CONVECTION_LINEAR_BYTES)
                                    : linear_order(base.N);
   const dim3 cgrid(launch_blocks(ord));
-  const bool nt = 2ull * TQ * sizeof(R) * base.N > LAST_LEVEL_BYTES;  // both population buffers
+  // Both population buffers above the last-level cache (168^3 FP32, 133^3 FP64):
+  // where diffusion starts to gain.  Runs of 16 steps, cached / streamed (us):
+  // FP32 160^3 632 / 755, 168^3 801 / 823, 170^3 895 / 892, 176^3 1028 / 959;
+  // FP64 128^3 681 / 861, 134^3 854 / 859, 136^3 944 / 959, 140^3 1098 / 991.
+  // Convection gains from a little below on (FP64 112^3 778 / 849, 120^3 1087 /
+  // 1055, 134^3 1498 / 1390; FP32 168^3 1431 / 1381, 176^3 1647 / 1517), the
+  // coupled loop too (five steps FP32 160^3 983 / 858, 170^3 1118 / 1056).
+  const bool nt = 2ull * TQ * sizeof(R) * base.N > LAST_LEVEL_BYTES;
   for (int n = 0; n < nsteps; ++n) {
     ThermalArgs a = base;
     a.ord = ord;
