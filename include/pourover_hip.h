@@ -12,8 +12,8 @@
  * context keeps a message readable with pol_last_error().  Work is enqueued
  * asynchronously on the hipStream_t passed as `stream` (NULL = legacy
  * default stream); only entry points that hand results back to host memory
- * (pol_reduce, pol_macroscopic / pol_step_ex / pol_step_from with a
- * reduction, pol_step_record with objective steps, pol_adjoint_collect,
+ * (pol_reduce, pol_macroscopic / pol_step_ex / pol_step_from /
+ * pol_coupled_step with a reduction, pol_step_record with objective steps, pol_adjoint_collect,
  * pol_field_stats, the thermal statistics, thermal steps with a stability
  * count or statistics) synchronise that stream.
  *
